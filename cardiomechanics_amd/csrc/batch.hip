@@ -34,6 +34,7 @@ struct cmg_batch {
     bool ptan = false;                             // surface-pressure tangent in the batched matrices
     DevBuf vals, dinv;                             // [S][nnzb*9], [S][N*9]
     DevBuf sw_inv, sw_y;                           // Schwarz: [S][sw_inv_len], [S][sw_y_len]
+    CoarseBuf coarse;                              // coarse correction of the Schwarz preconditioner
     bool schwarz = false;
     const int32_t* apply_skip = nullptr;           // sets the Schwarz application skips
     DevBuf cg_r, cg_z, cg_p, cg_q;                 // [S][n]
@@ -183,6 +184,7 @@ void bgather_tangent(cmg_batch* b) {
         ps.set_vals = c->nnzb * 9;
         ps.set_inv = c->sw_inv_len;
         ps.inv = b->sw_inv.p;
+        ps.coarse = &b->coarse;
         ps.flags = b->active.as<int32_t>();
         launch_patch_setup(c, b->vals.p, ps);
         return;
@@ -206,6 +208,7 @@ void batch_schwarz_apply(void* bb, const double* u, double* z) {
     ps.set_y = b->c->sw_y_len;
     ps.inv = b->sw_inv.p;
     ps.y = b->sw_y.as<double>();
+    ps.coarse = &b->coarse;
     ps.flags = b->apply_skip;
     launch_patch_apply(b->c, u, z, ps);
 }
@@ -274,8 +277,9 @@ int build_graph(cmg_batch* b) {
     return CMG_SUCCESS;
 }
 
-// CG on the sets flagged `solve` (already uploaded): delta = A^-1 rhs to rtol[s]
-int bcg_solve(cmg_batch* b, const std::vector<double>& rtol, std::vector<int32_t>& its) {
+// CG on the active sets (flags already uploaded): delta = A^-1 rhs to rtol[s]; done[s] = 2
+// where it broke down
+int bcg_run(cmg_batch* b, const std::vector<double>& rtol, std::vector<int32_t>& its, std::vector<int32_t>& done) {
     cmg_ctx* c = b->c;
     hipStream_t s = c->stream;
     const int S = b->S;
@@ -302,7 +306,29 @@ int bcg_solve(cmg_batch* b, const std::vector<double>& rtol, std::vector<int32_t
         if (all || total >= c->opt.krylov_maxit) break;
     }
     CMG_HIP_CHECK(hipGetLastError());
+    done.assign(b->h_int + S, b->h_int + 2 * S);
     its.assign(b->h_int + 2 * S, b->h_int + 3 * S);
+    return CMG_SUCCESS;
+}
+
+// bcg_run on the sets flagged `solve`; sets that break down with the coarse correction (it
+// finds the negative directions of an indefinite tangent at once) are solved again without it
+int bcg_solve(cmg_batch* b, const std::vector<double>& rtol, const std::vector<int32_t>& solve,
+              std::vector<int32_t>& its) {
+    const int S = b->S;
+    std::vector<int32_t> done;
+    CMG_TRY(upload_flags(b, solve));
+    CMG_TRY(bcg_run(b, rtol, its, done));
+    if (!b->schwarz || !b->c->coarse) return CMG_SUCCESS;
+    std::vector<int32_t> again(S, 0), its2;
+    for (int i = 0; i < S; i++) again[i] = solve[i] && done[i] == 2;
+    if (!any(again)) return CMG_SUCCESS;
+    for (int i = 0; i < S; i++)
+        if (again[i]) launch_fill_int(1, 1, b->coarse.bad.as<int>() + i, b->c->stream);
+    CMG_TRY(upload_flags(b, again));
+    CMG_TRY(bcg_run(b, rtol, its2, done));
+    for (int i = 0; i < S; i++)
+        if (again[i]) its[i] += its2[i];
     return CMG_SUCCESS;
 }
 
@@ -413,7 +439,7 @@ int bnewton(cmg_batch* b, double time, cmg_step_stats* st) {
         t_tan += now_s() - tb;
         const double tk = now_s();
         std::vector<int32_t> cits;
-        CMG_TRY(bcg_solve(b, eta_k, cits));
+        CMG_TRY(bcg_solve(b, eta_k, solve, cits));
         t_kry += now_s() - tk;
         std::vector<double> one(S, 0.0);
         for (int i = 0; i < S; i++)
@@ -502,8 +528,10 @@ int cmg_batch_create(cmg_ctx* c, int32_t n_sets, const cmg_material* materials, 
         // S sets of patch inverses (S x 548 MB in FP64 on the 200k LV): where they do not
         // fit, the batch keeps block Jacobi
         b->schwarz = b->sw_inv.alloc((size_t)S * c->sw_inv_len * kt) &&
-                     b->sw_y.alloc((size_t)S * c->sw_y_len * sizeof(double));
+                     b->sw_y.alloc((size_t)S * c->sw_y_len * sizeof(double)) &&
+                     (!c->coarse || b->coarse.alloc(c->co, S));
         if (!b->schwarz) {
+            b->coarse.release();
             b->sw_inv.release();
             b->sw_y.release();
             (void)hipGetLastError();   // the failed allocation is not an error of the batch

@@ -481,7 +481,10 @@ int cmg_create(const cmg_mesh* mesh, const cmg_material* materials, int32_t n_ma
         CMG_TRY(upload(c->mval, c->h_mval.data(), nnzb, s));
     }
     // -- preconditioner patches (need the block pattern)
-    if (c->opt.preconditioner != 1) CMG_TRY(build_vertex_patches(c.get(), mesh->elements));
+    if (c->opt.preconditioner != 1) {
+        CMG_TRY(build_vertex_patches(c.get(), mesh->elements));
+        if (c->schwarz) CMG_TRY(build_coarse(c.get(), mesh->ref_coords, mesh->elements));
+    }
     // -- surfaces
     c->h_pressure.assign(c->n_groups, 0.0);
     CMG_TRY(upload(c->pressure, c->h_pressure.data(), c->n_groups, s));
@@ -1133,9 +1136,26 @@ int bicgstab_device(cmg_ctx* c, const void* vals, const double* b, double* x, do
 
 int krylov(cmg_ctx* c, const void* vals, const double* b, double* x, double rtol, int maxit, cmg_solve_stats* st) {
     if (c->spmv_lanes == 0) CMG_TRY(tune_spmv(c, vals, b));
-    if (c->opt.krylov_method == 1) return bicgstab_device(c, vals, b, x, rtol, maxit, st);
-    if (c->opt.krylov_method == 2) return bicgstab(c, vals, b, x, rtol, maxit, st);
-    return gmres(c, vals, b, x, rtol, maxit, st);
+    auto solve = [&](cmg_solve_stats* ls) -> int {
+        if (c->opt.krylov_method == 1) return bicgstab_device(c, vals, b, x, rtol, maxit, ls);
+        if (c->opt.krylov_method == 2) return bicgstab(c, vals, b, x, rtol, maxit, ls);
+        return gmres(c, vals, b, x, rtol, maxit, ls);
+    };
+    CMG_TRY(solve(st));
+    if (!st->converged && c->schwarz && c->coarse && maxit > 0) {
+        // the coarse correction does not suit this matrix: once more without it, which then
+        // stays off until the preconditioner is built again
+        const int32_t reuse = c->opt.precond_reuse;
+        c->opt.precond_reuse = 1;
+        launch_fill_int(1, 1, c->co_buf.bad.as<int>(), c->stream);
+        launch_fill(c->n, 0.0, x, c->stream);
+        const int first = st->iterations;
+        const int rc = solve(st);
+        c->opt.precond_reuse = reuse;
+        CMG_TRY(rc);
+        st->iterations += first;
+    }
+    return CMG_SUCCESS;
 }
 
 // Cavity volume per pressure group at the device coordinates xd: the surface kernel's

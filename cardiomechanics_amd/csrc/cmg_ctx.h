@@ -32,6 +32,34 @@ struct DevBuf {
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
+// background grid of the coarse correction (coarse.hip) and the fine nodes' place in it
+struct CoarseGrid {
+    int nodes = 0, ld = 0;              // grid nodes, leading dimension of A_c (3 nodes, padded)
+    int nx = 0, ny = 0, nz = 0;         // cells per axis
+    int n_chunk = 0, n_rchunk = 0;
+    int64_t set_A = 0;                  // ld * ld
+    const int32_t* pos = nullptr;       // [N] cell of each fine node, 10 bits per axis
+    const double* frac = nullptr;       // [N][3] position within the cell, 0..1
+    const int32_t* order = nullptr;     // [N] fine nodes sorted by cell
+    const int32_t* cell = nullptr;      // [N] index of the node's cell among the occupied ones
+    const int32_t* corner = nullptr;    // [cells][8] grid nodes of each occupied cell
+    const int32_t* chunk = nullptr;     // [n_chunk][3] cell, first entry of order, length (Galerkin product)
+    const int32_t* rchunk = nullptr;    // [n_rchunk][3] the same for the restriction
+    const int32_t* map = nullptr;       // grid position -> grid node or -1
+    const int32_t* ijk = nullptr;       // [nodes] grid position, 10 bits per axis
+    const int32_t *gptr = nullptr, *gidx = nullptr;   // per grid node: 8 chunk + corner, in chunk order
+    const int32_t* rptr = nullptr;      // per grid node: its run of restriction partials
+    const int32_t* rslot = nullptr;     // [8 n_rchunk] place of each chunk's corner in those runs
+};
+
+// dense coarse matrices of S sets (inverted in place) and the scratch of their setup and use
+struct CoarseBuf {
+    DevBuf A, diag, U, C, gpart, rpart, rc, zc;
+    DevBuf bad;   // [S] 1: the correction is off (A_c was not positive, or a solve failed with it)
+    bool alloc(const CoarseGrid& g, int S);
+    void release();
+};
+
 int fail(const std::string& m, int code = CMG_ERR_INVALID);
 int to_dev_material(const cmg_material& m, DevMaterial& d);   // validates the law
 int alloc(DevBuf& b, size_t bytes);
@@ -143,6 +171,12 @@ struct cmg_ctx {
     int64_t sw_n_small = 0;
     int sw_nd_small = 0;
     int64_t sw_inv_len = 0, sw_y_len = 0;   // inverse values and patch-vector rows of all patches
+    // coarse-grid correction of the Schwarz preconditioner (coarse.hip)
+    bool coarse = false;
+    cmg::CoarseGrid co;
+    cmg::DevBuf co_pos, co_frac, co_order, co_cell, co_corner, co_chunk, co_rchunk, co_map, co_ijk;
+    cmg::DevBuf co_gptr, co_gidx, co_rptr, co_rslot;
+    cmg::CoarseBuf co_buf;
 };
 
 namespace cmg {
@@ -161,8 +195,15 @@ struct PatchSets {
     int64_t set_vals = 0, set_inv = 0, set_vec = 0, set_y = 0;
     void* inv = nullptr;        // [S][sw_inv_len] (the context's sw_inv when null)
     double* y = nullptr;        // [S][sw_y_len] (the context's sw_y when null)
+    CoarseBuf* coarse = nullptr;    // coarse matrices of the sets (the context's co_buf when null)
     const int32_t* flags = nullptr;
 };
+// coarse-grid correction (coarse.hip): grid nodes at most, the grid of a context with patches
+// (sets c->coarse), the inverse of A_c from the block values, z_c = A_c^-1 r_c
+constexpr int kCoarseMaxNodes = 340;
+int build_coarse(cmg_ctx* c, const double* coords, const int32_t* elements);
+void launch_coarse_setup(cmg_ctx* c, const void* vals, const PatchSets& ps);
+void launch_coarse_solve(cmg_ctx* c, const PatchSets& ps);
 void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps = PatchSets());  // patch inverses
 // z = sum_p R_p^T A_p^-1 R_p r
 void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets& ps = PatchSets());

@@ -14,7 +14,7 @@
 // the inverse column-major (FP64, or FP32 in mixed precision).  Per application: one
 // wave per patch forms y_p = A_p^{-1} r_p (lane i owns row i: coalesced column reads),
 // then every node sums its one or two patch results in patch order (deterministic,
-// no atomics).
+// no atomics) and the coarse-grid correction (coarse.hip).
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -136,9 +136,45 @@ __global__ __launch_bounds__(kWave) void k_patch_setup(int64_t n, const int32_t*
         for (int i = lane; i < nd; i += kWave) out[(int64_t)j * nd + i] = (IT)A[i * nd + j];
 }
 
-// y_p = A_p^{-1} r_p, one wave per patch, four patches per workgroup
+// restriction partials of one chunk of fine nodes (all of one grid cell): [corner][component],
+// summed over the workgroup in a fixed order
+template <typename F>
+__device__ __forceinline__ void restrict_chunk(const CoarseGrid& g, int ch, const uint8_t* bcmask, F rhs, double* out,
+                                               double* sh) {
+    const int start = g.rchunk[3 * ch + 1], count = g.rchunk[3 * ch + 2];
+    double s[24];
+#pragma unroll
+    for (int q = 0; q < 24; q++) s[q] = 0.0;
+    for (int k = (int)threadIdx.x; k < count; k += 256) {
+        const int64_t n = g.order[start + k];
+        const int m = bcmask[n];
+        const double fx = g.frac[3 * n], fy = g.frac[3 * n + 1], fz = g.frac[3 * n + 2];
+        const double v[3] = {(m & 1) ? 0.0 : rhs(3 * n), (m & 2) ? 0.0 : rhs(3 * n + 1),
+                             (m & 4) ? 0.0 : rhs(3 * n + 2)};
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            const double w = ((a & 1) ? fx : 1.0 - fx) * ((a & 2) ? fy : 1.0 - fy) * ((a & 4) ? fz : 1.0 - fz);
+#pragma unroll
+            for (int i = 0; i < 3; i++) s[3 * a + i] += w * v[i];
+        }
+    }
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+#pragma unroll
+    for (int q = 0; q < 24; q++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s[q] += __shfl_xor(s[q], o, 64);
+        if (lane == 0) sh[24 * w + q] = s[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < 24)
+        out[3 * (int64_t)g.rslot[8 * ch + threadIdx.x / 3] + threadIdx.x % 3] = sh[threadIdx.x] + sh[24 + threadIdx.x] + sh[48 + threadIdx.x] + sh[72 + threadIdx.x];
+}
+
+// y_p = A_p^{-1} r_p, one wave per patch, four patches per workgroup; the first g.n_rchunk
+// workgroups restrict r to the coarse grid instead
 template <typename IT>
-__global__ __launch_bounds__(256) void k_patch_apply(int64_t P, const int32_t* pptr, const int32_t* pnodes,
+__global__ __launch_bounds__(256) void k_patch_apply(CoarseGrid g, const uint8_t* bcmask, double* rpart,
+                                                     int64_t set_rpart, int64_t P, const int32_t* pptr, const int32_t* pnodes,
                                                      const int64_t* iptr, const IT* inv, const double* r,
                                                      double* y, int nd_max, int64_t set_inv, int64_t set_vec,
                                                      int64_t set_y, const int32_t* skip) {
@@ -148,13 +184,18 @@ __global__ __launch_bounds__(256) void k_patch_apply(int64_t P, const int32_t* p
     inv += set * set_inv;
     r += set * set_vec;
     y += set * set_y;
+    auto rhs = [&](int64_t i) { return r[i]; };
+    if ((int)blockIdx.x < g.n_rchunk) {
+        restrict_chunk(g, (int)blockIdx.x, bcmask, rhs, rpart + set * set_rpart, lds);
+        return;
+    }
     const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int64_t p = (int64_t)blockIdx.x * 4 + w;
+    const int64_t p = ((int64_t)blockIdx.x - g.n_rchunk) * 4 + w;
     double* rp = lds + (size_t)w * nd_max;
     const bool valid = p < P;
     const int p0 = valid ? pptr[p] : 0;
     const int nd = valid ? 3 * (pptr[p + 1] - p0) : 0;
-    for (int l = lane; l < nd; l += kWave) rp[l] = r[3 * (int64_t)pnodes[p0 + l / 3] + l % 3];
+    for (int l = lane; l < nd; l += kWave) rp[l] = rhs(3 * (int64_t)pnodes[p0 + l / 3] + l % 3);
     __syncthreads();
     if (!valid) return;
     const IT* a = inv + iptr[p];
@@ -166,8 +207,9 @@ __global__ __launch_bounds__(256) void k_patch_apply(int64_t P, const int32_t* p
     }
 }
 
-// z[3n + c] = sum over the patches holding node n of their y rows, in patch order
-__global__ __launch_bounds__(256) void k_patch_gather(int64_t N, const int32_t* cptr, const int32_t* cpos,
+// z[3n + c] = sum over the patches holding node n of their y rows, in patch order, plus the
+// coarse correction at the node (g.nodes > 0)
+__global__ __launch_bounds__(256) void k_patch_gather(CoarseGrid g, const uint8_t* bcmask, const double* zc, int64_t N, const int32_t* cptr, const int32_t* cpos,
                                                       const double* y, double* z, int64_t set_y, int64_t set_vec,
                                                       const int32_t* skip) {
     const int64_t set = blockIdx.y;
@@ -182,6 +224,24 @@ __global__ __launch_bounds__(256) void k_patch_gather(int64_t N, const int32_t* 
         s0 += q[0];
         s1 += q[1];
         s2 += q[2];
+    }
+    if (g.nodes > 0) {
+        const int32_t* ids = g.corner + 8 * (int64_t)g.cell[n];
+        const double fx = g.frac[3 * n], fy = g.frac[3 * n + 1], fz = g.frac[3 * n + 2];
+        const double* u = zc + set * (int64_t)g.ld;
+        double c0 = 0.0, c1 = 0.0, c2 = 0.0;
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            const double w = ((a & 1) ? fx : 1.0 - fx) * ((a & 2) ? fy : 1.0 - fy) * ((a & 4) ? fz : 1.0 - fz);
+            const double* q = u + 3 * ids[a];
+            c0 += w * q[0];
+            c1 += w * q[1];
+            c2 += w * q[2];
+        }
+        const int m = bcmask[n];
+        s0 += (m & 1) ? 0.0 : c0;
+        s1 += (m & 2) ? 0.0 : c1;
+        s2 += (m & 4) ? 0.0 : c2;
     }
     z[3 * n] = s0;
     z[3 * n + 1] = s1;
@@ -296,24 +356,32 @@ void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps) {
             CMG_PSETUP(double, double);
 #undef CMG_PSETUP
     }
+    if (c->coarse) launch_coarse_setup(c, vals, ps);
 }
 
 void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets& ps) {
     const int ndm = c->sw_nd_max;
-    const dim3 grid((unsigned)((c->sw_P + 3) / 4), ps.S);
-    const size_t lds = (size_t)4 * ndm * sizeof(double);
+    const CoarseGrid g = c->coarse ? c->co : CoarseGrid();
+    const CoarseBuf& cb = ps.coarse ? *ps.coarse : c->co_buf;
+    const int64_t set_rpart = (int64_t)g.n_rchunk * 24;
+    const uint8_t* bc = c->bcmask.as<uint8_t>();
+    const dim3 grid((unsigned)((c->sw_P + 3) / 4) + (unsigned)g.n_rchunk, ps.S);
+    const size_t lds = (size_t)std::max(4 * ndm, 96) * sizeof(double);
     const void* inv = ps.inv ? ps.inv : c->sw_inv.p;
     double* y = ps.y ? ps.y : c->sw_y.as<double>();
+#define CMG_PAPPLY(IT)                                                                                              \
+    hipLaunchKernelGGL(k_patch_apply<IT>, grid, dim3(256), lds, c->stream, g, bc, cb.rpart.as<double>(), set_rpart, \
+                       c->sw_P, c->sw_pptr.as<int32_t>(), c->sw_pnodes.as<int32_t>(), c->sw_iptr.as<int64_t>(),     \
+                       (const IT*)inv, r, y, ndm, ps.set_inv, ps.set_vec, ps.set_y, ps.flags)
     if (c->fp32)
-        hipLaunchKernelGGL(k_patch_apply<float>, grid, dim3(256), lds, c->stream, c->sw_P, c->sw_pptr.as<int32_t>(),
-                           c->sw_pnodes.as<int32_t>(), c->sw_iptr.as<int64_t>(), (const float*)inv, r, y, ndm,
-                           ps.set_inv, ps.set_vec, ps.set_y, ps.flags);
+        CMG_PAPPLY(float);
     else
-        hipLaunchKernelGGL(k_patch_apply<double>, grid, dim3(256), lds, c->stream, c->sw_P, c->sw_pptr.as<int32_t>(),
-                           c->sw_pnodes.as<int32_t>(), c->sw_iptr.as<int64_t>(), (const double*)inv, r, y, ndm,
-                           ps.set_inv, ps.set_vec, ps.set_y, ps.flags);
-    hipLaunchKernelGGL(k_patch_gather, dim3((unsigned)((c->N + 255) / 256), ps.S), dim3(256), 0, c->stream, c->N,
-                       c->sw_cptr.as<int32_t>(), c->sw_cpos.as<int32_t>(), y, z, ps.set_y, ps.set_vec, ps.flags);
+        CMG_PAPPLY(double);
+#undef CMG_PAPPLY
+    if (c->coarse) launch_coarse_solve(c, ps);
+    hipLaunchKernelGGL(k_patch_gather, dim3((unsigned)((c->N + 255) / 256), ps.S), dim3(256), 0, c->stream, g, bc,
+                       cb.zc.as<double>(), c->N, c->sw_cptr.as<int32_t>(), c->sw_cpos.as<int32_t>(), y, z, ps.set_y,
+                       ps.set_vec, ps.flags);
 }
 
 }  // namespace cmg

@@ -149,8 +149,9 @@ typedef struct cmg_options {
                                    857-866); off when both are 0 */
     int32_t preconditioner;     /* of the Krylov solves: 1 3x3 nodal block Jacobi, 2 vertex-patch
                                    additive Schwarz (T10: each element vertex with the midside
-                                   nodes of its edges, patch matrices inverted on the device;
-                                   block Jacobi for T4); 0 (default):
+                                   nodes of its edges, patch matrices inverted on the device,
+                                   plus a coarse-grid correction over the trilinear hats of a
+                                   background grid; block Jacobi for T4); 0 (default):
                                    2 where it applies */
     int32_t precond_reuse;      /* 1 (default): the Schwarz preconditioner is built from the first
                                    tangent of each Newton solve and reused by its later linear solves
@@ -353,8 +354,8 @@ int cmg_set_land17_state(cmg_ctx* ctx, const double* state, double commit_time);
  * copies of a context's quasi-static problem with their own material tables, one
  * mesh.  Each set follows cmg_static_step (CBSolverEquilibrium.cpp:234-363);
  * every kernel launch covers all sets, and the linear solve is a conjugate gradient,
- * preconditioned like the context's solves (vertex-patch Schwarz with one set of patch
- * inverses per parameter set, or 3x3 block Jacobi), whose scalars stay on the device
+ * preconditioned like the context's solves (vertex-patch Schwarz and coarse correction
+ * with one set of inverses per parameter set, or 3x3 block Jacobi), whose scalars stay on the device
  * (runs of iterations are replayed as one HIP graph).  CG needs symmetric matrices: the
  * assembled follower-pressure tangent of a closed T3 cavity whose rim is clamped
  * (the LV endocardium) is symmetric and is included when the context's
