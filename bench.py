@@ -54,8 +54,8 @@ def main():
     ap.add_argument("--beat-runs", default="fp64_bj,fp64,mixed,mixed_warm",
                     help="comma list of fp64_bj (block Jacobi), fp64, mixed, mixed_warm (vertex-patch Schwarz)")
     ap.add_argument("--krylov-method", type=int, default=None,
-                    help="Krylov solver of the beat window runs (0 GMRES, 1 BiCGStab with device-side scalars, "
-                         "2 BiCGStab with host-side scalars; default: the library's)")
+                    help="Krylov solver of the beat window runs (0 GMRES, 1 or 2 BiCGStab; "
+                         "default: the library's)")
     ap.add_argument("--precond-reuse", type=int, default=None,
                     help="1: the beat window runs build the preconditioner once per Newton solve (default: the "
                          "library's)")

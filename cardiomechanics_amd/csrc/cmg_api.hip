@@ -13,7 +13,6 @@
 #include <string>
 #include <vector>
 
-#include "batch_kernels.h"
 #include "cmg_ctx.h"
 #include "land17_calcium.h"
 
@@ -173,7 +172,7 @@ void cmg_default_options(cmg_options* o) {
     o->newton_maxit = 50;
     o->krylov_restart = 80;
     o->krylov_maxit = 4000;
-    o->krylov_method = 2;   // BiCGStab, host-side scalars: the fastest on the 200k-element LV beat
+    o->krylov_method = 2;   // BiCGStab
     o->device = 0;
     o->element_variant = 0;   // by precision: 6 (FP64), 5 (mixed), the fastest of each on the LV
     o->newton_atol = 1e-8;
@@ -203,7 +202,7 @@ void cmg_destroy(cmg_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->bicg_graph) (void)hipGraphExecDestroy(c->bicg_graph);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
-    if (c->h_part) (void)hipHostFree(c->h_part);
+    if (c->bicg_host) (void)hipHostFree(c->bicg_host);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -848,112 +847,6 @@ int gmres(cmg_ctx* c, const void* vals, const double* b, double* x, double rtol,
 }
 
 
-// BiCGStab with right preconditioning (van der Vorst 1992).  Two host
-// synchronisations per iteration: (r^, v) for alpha, and one fused fetch of
-// (r^,t) (s,t) (t,t) (r^,s) (s,s) from which omega, the next rho and the updated
-// residual norm ||s - omega t|| follow without another pass.
-int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, double rtol, int maxit, cmg_solve_stats* st) {
-    hipStream_t s = c->stream;
-    const int64_t n = c->n;
-    const int nb = dot_blocks(n);
-    double* W = c->gm_V.as<double>();   // (restart + 2) >= 10 vectors
-    double* rh = W;
-    double* sv = W + n;
-    double* t = W + 2 * n;
-    double* r = W + 3 * n;
-    double* p = W + 4 * n;
-    double* v = W + 5 * n;
-    double* ph = W + 6 * n;
-    double* sh = W + 7 * n;
-    double* part = c->gm_partial.as<double>();
-    const double* dinv = c->dinv.as<double>();
-    const int64_t* rp = c->rowptr.as<int64_t>();
-    const int32_t* ci = c->colind.as<int32_t>();
-    if (c->h_part_len < 5 * (int64_t)nb) {
-        if (c->h_part) CMG_HIP_CHECK(hipHostFree(c->h_part));
-        c->h_part = nullptr;
-        CMG_HIP_CHECK(hipHostMalloc((void**)&c->h_part, 5 * (size_t)nb * sizeof(double), hipHostMallocDefault));
-        c->h_part_len = 5 * (int64_t)nb;
-    }
-    // dot products: per-chunk partials copied to the host and summed there in chunk order
-    auto host_sums = [&](int k, double* out) -> int {
-        CMG_HIP_CHECK(hipMemcpyAsync(c->h_part, part, (size_t)k * nb * sizeof(double), hipMemcpyDeviceToHost, s));
-        CMG_HIP_CHECK(hipStreamSynchronize(s));
-        for (int j = 0; j < k; j++) out[j] = 0.0;
-        for (int blk = 0; blk < nb; blk++)
-            for (int j = 0; j < k; j++) out[j] += c->h_part[(int64_t)blk * k + j];
-        return CMG_SUCCESS;
-    };
-    const bool sw = use_schwarz(c);
-    precond_setup(c, vals);
-    double bnorm;
-    CMG_TRY(norm2(c, b, &bnorm));
-    launch_spmv(c->N, rp, ci, vals, c->fp32, x, v, s, c->spmv_lanes, c->spmv_layout);
-    launch_waxpby(n, 1.0, b, -1.0, v, r, s);
-    double rn;
-    CMG_TRY(norm2(c, r, &rn));
-    st->initial_residual = rn;
-    st->iterations = 0;
-    st->converged = 0;
-    const double target = rtol * (bnorm > 0 ? bnorm : 1.0);
-    if (rn <= target || rn == 0.0) {
-        st->final_residual = rn;
-        st->converged = 1;
-        return CMG_SUCCESS;
-    }
-    int it = 0, restarts = 0;
-    bool fresh = true;
-    double rho = 1.0, alpha = 1.0, omega = 1.0, rho_new = rn * rn;
-    while (it < maxit) {
-        // p = r + beta (p - omega v) (p = r on a (re)start, with shadow residual r^ = r); ph = D^-1 p
-        double beta = 0.0;
-        if (fresh) {
-            launch_scale_copy(n, 1.0, r, rh, s);
-            rho_new = rn * rn;
-        } else {
-            beta = (rho_new / rho) * (alpha / omega);
-        }
-        launch_bicg_p_bj(c->N, fresh, beta, omega, r, v, sw ? nullptr : dinv, p, ph, s);
-        if (sw) precond_apply(c, p, ph);
-        fresh = false;
-        rho = rho_new;
-        launch_spmv(c->N, rp, ci, vals, c->fp32, ph, v, s, c->spmv_lanes, c->spmv_layout);
-        launch_multidot(n, 1, rh, 0, v, part, s);
-        double d0;
-        CMG_TRY(host_sums(1, &d0));
-        bool breakdown = !(std::fabs(d0) > 0.0) || !std::isfinite(d0);
-        if (!breakdown) {
-            alpha = rho / d0;
-            launch_bicg_s_bj(c->N, alpha, r, v, sw ? nullptr : dinv, sv, sh, s);   // s = r - alpha v, sh = D^-1 s
-            if (sw) precond_apply(c, sv, sh);
-            launch_spmv(c->N, rp, ci, vals, c->fp32, sh, t, s, c->spmv_lanes, c->spmv_layout);
-            launch_bicg_dots5(n, rh, sv, t, part, s);              // (rh,t) (s,t) (t,t) (rh,s) (s,s)
-            double d5[5];
-            CMG_TRY(host_sums(5, d5));
-            const double rt = d5[0], st_ = d5[1], tt = d5[2], rs = d5[3], ss = d5[4];
-            omega = tt > 0.0 ? st_ / tt : 0.0;
-            launch_bicg_xr(n, alpha, omega, ph, sh, sv, t, x, r, s);   // x += alpha ph + omega sh, r = s - omega t
-            it++;
-            rn = std::sqrt(std::max(ss - 2.0 * omega * st_ + omega * omega * tt, 0.0));
-            rho_new = rs - omega * rt;
-            breakdown = omega == 0.0 || !(std::fabs(rho_new) > 0.0) || !std::isfinite(rn);
-        }
-        if (rn <= target || breakdown) {
-            // the recurrence residual drifts from b - A x: confirm, restart if needed
-            launch_spmv(c->N, rp, ci, vals, c->fp32, x, v, s, c->spmv_lanes, c->spmv_layout);
-            launch_waxpby(n, 1.0, b, -1.0, v, r, s);
-            CMG_TRY(norm2(c, r, &rn));
-            if (rn <= target || ++restarts > 50 || !std::isfinite(rn)) break;
-            fresh = true;
-        }
-    }
-    st->iterations = it;
-    st->final_residual = rn;
-    st->converged = rn <= target;
-    CMG_HIP_CHECK(hipGetLastError());
-    return CMG_SUCCESS;
-}
-
 // SpMV layout: the fastest of 4 / 8 / 16 lanes per block row, one block or one
 // 144-byte chunk per step, on this matrix (HIP events, one warm and two timed products
 // each), chosen once per context
@@ -963,15 +856,13 @@ int tune_spmv(cmg_ctx* c, const void* vals, const double* b) {
     CMG_HIP_CHECK(hipEventCreate(&e0));
     CMG_HIP_CHECK(hipEventCreate(&e1));
     const int lanes[3][3] = {{4, 8, 16}, {4, 8, 16}, {16, 32, 64}};
-    float best = 1e30f, best_blk = 1e30f;
+    float best = 1e30f;
     const int64_t* rp = c->rowptr.as<int64_t>();
     const int32_t* ci = c->colind.as<int32_t>();
     if (c->opt.spmv_choice >= 1 && c->opt.spmv_choice <= 9) {   // fixed by the caller, no timing
         const int layout = (c->opt.spmv_choice - 1) / 3, li = (c->opt.spmv_choice - 1) % 3;
         c->spmv_lanes = lanes[layout][li];
         c->spmv_layout = layout;
-        c->bicg_lanes = layout == kSpmvFlat ? 16 : lanes[layout][li];
-        c->bicg_chunked = layout == kSpmvChunk;
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         return CMG_SUCCESS;
@@ -992,11 +883,6 @@ int tune_spmv(cmg_ctx* c, const void* vals, const double* b) {
                 c->spmv_lanes = l;
                 c->spmv_layout = layout;
             }
-            if (layout != kSpmvFlat && ms < best_blk) {
-                best_blk = ms;
-                c->bicg_lanes = l;
-                c->bicg_chunked = layout == kSpmvChunk;
-            }
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -1004,153 +890,26 @@ int tune_spmv(cmg_ctx* c, const void* vals, const double* b) {
 }
 
 
-// BiCGStab with the scalar recurrences on the device (BatchBiCG with one set): an
-// iteration is eight launches without host synchronisation; `bicg_chunk` iterations
-// are replayed as one HIP graph, after which the host reads the done flag.  A
-// converged or broken-down recurrence is confirmed with the true residual b - A x
-// and restarted from the current x when needed.
-int bicgstab_device(cmg_ctx* c, const void* vals, const double* b, double* x, double rtol, int maxit,
-                    cmg_solve_stats* st) {
-    hipStream_t s = c->stream;
-    const int64_t n = c->n;
-    const int64_t* rp = c->rowptr.as<int64_t>();
-    const int32_t* ci = c->colind.as<int32_t>();
-    precond_setup(c, vals);
-    if (!c->bicg_part.p) {
-        CMG_TRY(alloc(c->bicg_part, (size_t)bicg_part_ld(c->N) * sizeof(double)));
-        CMG_TRY(alloc(c->bicg_sc, 16 * sizeof(double)));
-        CMG_TRY(alloc(c->bicg_flags, 8 * sizeof(int32_t)));
-    }
-    double* W = c->gm_V.as<double>();   // >= 10 work vectors
-    BatchBiCG k;
-    k.S = 1;
-    k.x = x;
-    k.r = W;
-    k.rh = W + n;
-    k.p = W + 2 * n;
-    k.v = W + 3 * n;
-    k.s = W + 4 * n;
-    k.t = W + 5 * n;
-    k.ph = W + 6 * n;
-    k.sh = W + 7 * n;
-    double* sc = c->bicg_sc.as<double>();
-    k.rho = sc;
-    k.alpha = sc + 1;
-    k.omega = sc + 2;
-    k.beta = sc + 3;
-    k.rr = sc + 4;
-    k.tol2 = sc + 5;
-    double* rtol_dev = sc + 6;
-    int32_t* fl = c->bicg_flags.as<int32_t>();
-    k.done = fl;
-    k.it = fl + 1;
-    k.fin = fl + 2;
-    int32_t* active = fl + 3;
-    k.part = c->bicg_part.as<double>();
-    k.part_ld = bicg_part_ld(c->N);
-    launch_fill(1, rtol, rtol_dev, s);
-    launch_fill_int(4, 0, fl, s);
-    launch_fill_int(1, 1, active, s);
-    auto restart = [&]() {
-        // r = b - A x, then r^ = r, p = r and the scalars
-        launch_spmv(c->N, rp, ci, vals, c->fp32, x, k.r, s, c->spmv_lanes, c->spmv_layout);
-        launch_waxpby(n, 1.0, b, -1.0, k.r, k.r, s);
-        launch_bicg_init(k, c->N, b, rtol_dev, active, s);
-    };
-    restart();
-    // Schwarz: the patch kernels skip, like the update kernels, once the recurrence has
-    // finished within a replayed chunk (the done flag k.done)
-    const PrecondApply apply = use_schwarz(c) ? [](void* cc, const double* u, double* z) {
-        cmg_ctx* cx = static_cast<cmg_ctx*>(cc);
-        PatchSets ps;
-        ps.flags = cx->bicg_flags.as<int32_t>();
-        launch_patch_apply(cx, u, z, ps);
-    } : PrecondApply(nullptr);
-    auto iterate = [&]() {
-        launch_bicg_iteration(k, c->bicg_lanes, c->bicg_chunked, c->N, rp, ci, vals, c->fp32, 0,
-                              c->dinv.as<double>(), s, apply, c);
-    };
-    const bool graph_ok = c->bicg_graph != nullptr && c->bicg_graph_x == x && c->bicg_graph_vals == vals;
-    if (!graph_ok && c->bicg_use_graph) {
-        if (c->bicg_graph) (void)hipGraphExecDestroy(c->bicg_graph);
-        c->bicg_graph = nullptr;
-        hipGraph_t g = nullptr;
-        CMG_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        for (int i = 0; i < c->bicg_chunk; i++) iterate();
-        CMG_HIP_CHECK(hipStreamEndCapture(s, &g));
-        hipError_t e = hipGraphInstantiate(&c->bicg_graph, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        CMG_HIP_CHECK(e);
-        c->bicg_graph_x = x;
-        c->bicg_graph_vals = vals;
-    }
-    double* hd = c->h_pinned + 3500;   // pinned staging beyond the GMRES areas
-    int32_t* hi = reinterpret_cast<int32_t*>(c->h_pinned + 3600);
-    CMG_HIP_CHECK(hipMemcpyAsync(hd, sc, 6 * sizeof(double), hipMemcpyDeviceToHost, s));
-    CMG_HIP_CHECK(hipStreamSynchronize(s));
-    const double target = std::sqrt(std::max(hd[5], 0.0));
-    double rn = std::sqrt(std::max(hd[4], 0.0));
-    st->initial_residual = rn;
-    st->iterations = 0;
-    st->converged = 0;
-    int restarts = 0;
-    if (rn <= target) {
-        st->final_residual = rn;
-        st->converged = 1;
-        return CMG_SUCCESS;
-    }
-    for (;;) {
-        if (c->bicg_graph)
-            CMG_HIP_CHECK(hipGraphLaunch(c->bicg_graph, s));
-        else
-            for (int i = 0; i < c->bicg_chunk; i++) iterate();
-        CMG_HIP_CHECK(hipMemcpyAsync(hi, fl, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        CMG_HIP_CHECK(hipStreamSynchronize(s));
-        const int done = hi[0], its = hi[1];
-        st->iterations = its;
-        if (done == 0) {
-            if (its >= maxit) break;
-            continue;
-        }
-        // confirm with the true residual (the recurrence drifts from b - A x)
-        launch_spmv(c->N, rp, ci, vals, c->fp32, x, k.r, s, c->spmv_lanes, c->spmv_layout);
-        launch_waxpby(n, 1.0, b, -1.0, k.r, k.r, s);
-        CMG_TRY(norm2(c, k.r, &rn));
-        if (rn <= target) {
-            st->converged = 1;
-            break;
-        }
-        if (++restarts > 50 || its >= maxit || !std::isfinite(rn)) break;
-        launch_fill_int(1, 0, k.done, s);
-        launch_bicg_init(k, c->N, b, rtol_dev, active, s);   // restart from the current x
-    }
-    if (!st->converged) {   // final residual of an unconverged solve
-        launch_spmv(c->N, rp, ci, vals, c->fp32, x, k.r, s, c->spmv_lanes, c->spmv_layout);
-        launch_waxpby(n, 1.0, b, -1.0, k.r, k.r, s);
-        CMG_TRY(norm2(c, k.r, &rn));
-    }
-    st->final_residual = rn;
-    CMG_HIP_CHECK(hipGetLastError());
-    return CMG_SUCCESS;
-}
-
-int krylov(cmg_ctx* c, const void* vals, const double* b, double* x, double rtol, int maxit, cmg_solve_stats* st) {
+int krylov(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero_guess, double rtol, int maxit,
+           cmg_solve_stats* st) {
     if (c->spmv_lanes == 0) CMG_TRY(tune_spmv(c, vals, b));
-    auto solve = [&](cmg_solve_stats* ls) -> int {
-        if (c->opt.krylov_method == 1) return bicgstab_device(c, vals, b, x, rtol, maxit, ls);
-        if (c->opt.krylov_method == 2) return bicgstab(c, vals, b, x, rtol, maxit, ls);
+    auto solve = [&](bool zero, cmg_solve_stats* ls) -> int {
+        if (c->opt.krylov_method == 1 || c->opt.krylov_method == 2) {
+            precond_setup(c, vals);
+            return bicgstab(c, vals, b, x, zero, rtol, maxit, ls);
+        }
+        if (zero) launch_fill(c->n, 0.0, x, c->stream);
         return gmres(c, vals, b, x, rtol, maxit, ls);
     };
-    CMG_TRY(solve(st));
+    CMG_TRY(solve(zero_guess, st));
     if (!st->converged && c->schwarz && c->coarse && maxit > 0) {
         // the coarse correction does not suit this matrix: once more without it, which then
         // stays off until the preconditioner is built again
         const int32_t reuse = c->opt.precond_reuse;
         c->opt.precond_reuse = 1;
         launch_fill_int(1, 1, c->co_buf.bad.as<int>(), c->stream);
-        launch_fill(c->n, 0.0, x, c->stream);
         const int first = st->iterations;
-        const int rc = solve(st);
+        const int rc = solve(true, st);
         c->opt.precond_reuse = reuse;
         CMG_TRY(rc);
         st->iterations += first;
@@ -1381,7 +1140,7 @@ int cmg_linear_solve(cmg_ctx* c, const double* values, const double* b, double* 
     cmg_solve_stats local;
     if (!st) st = &local;
     c->precond_built = false;   // a standalone solve always builds from its own matrix
-    CMG_TRY(krylov(c, c->vals.p, c->r.as<double>(), c->delta.as<double>(), rtol, c->opt.krylov_maxit, st));
+    CMG_TRY(krylov(c, c->vals.p, c->r.as<double>(), c->delta.as<double>(), false, rtol, c->opt.krylov_maxit, st));
     CMG_HIP_CHECK(hipMemcpyAsync(x, c->delta.p, vb, hipMemcpyDeviceToHost, c->stream));
     CMG_HIP_CHECK(hipStreamSynchronize(c->stream));
     return st->converged ? CMG_SUCCESS : CMG_FAILED;
@@ -1632,9 +1391,8 @@ int newton(cmg_ctx* c, double time, double cm, double cd, cmg_step_stats* st) {
         t_tan += now_s() - tb;
         const double tk = now_s();
         launch_scale_copy(n, -1.0, r, c->dsave.as<double>(), s);
-        launch_fill(n, 0.0, delta, s);
         cmg_solve_stats ls;
-        CMG_TRY(krylov(c, c->vals.p, c->dsave.as<double>(), delta, eta_k, c->opt.krylov_maxit, &ls));
+        CMG_TRY(krylov(c, c->vals.p, c->dsave.as<double>(), delta, true, eta_k, c->opt.krylov_maxit, &ls));
         kry_total += ls.iterations;
         t_kry += now_s() - tk;
         if (c->trace)

@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 
+#include "bicgstab.h"
 #include "cmg_internal.h"
 
 namespace cmg {
@@ -90,17 +91,13 @@ struct cmg_ctx {
     int n_mats = 0;
     int spmv_lanes = 0;         // lanes per block row of the SpMV, 0 until timed on the first solve
     int spmv_layout = 0;        // kSpmvBlock / kSpmvChunk / kSpmvFlat
-    // the fastest block or chunk layout: the device-scalar BiCGStab fuses its SpMV with
-    // dot products and exists in those two layouts only
-    int bicg_lanes = 8;
-    bool bicg_chunked = false;
-    // device-scalar BiCGStab: workspace and the graph of `bicg_chunk` iterations
-    cmg::DevBuf bicg_part, bicg_sc, bicg_flags;
+    // BiCGStab: partial sums, scalars, the word the host follows, the graph of a few iterations
+    cmg::DevBuf bicg_part, bicg_sc;
+    cmg::BicgHost* bicg_host = nullptr;
+    unsigned bicg_seq = 0;
     hipGraphExec_t bicg_graph = nullptr;
     const void* bicg_graph_x = nullptr;
     const void* bicg_graph_vals = nullptr;
-    int bicg_chunk = 16;
-    bool bicg_use_graph = true;
     double spmv_ms[9] = {};     // timed SpMV: block at 4/8/16 lanes, chunks at 4/8/16, flat at 16/32/64
     bool fp32 = false;
     bool trace = false;         // CMG_NEWTON_TRACE: one stderr line per Newton iteration
@@ -137,8 +134,6 @@ struct cmg_ctx {
     cmg::DevBuf gm_V, gm_partial, gm_h, gm_y;
     int gm_m = 0;
     double* h_pinned = nullptr;   // host staging for reductions
-    double* h_part = nullptr;     // host staging for per-chunk dot partials (BiCGStab), 5 per chunk
-    int64_t h_part_len = 0;
     cmg::DevBuf corrupt;
     // static solver bookkeeping (CBSolverEquilibrium::UpdateInitialGuess)
     double time_last = 0.0, step_last = 0.0;
@@ -207,4 +202,10 @@ void launch_coarse_solve(cmg_ctx* c, const PatchSets& ps);
 void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps = PatchSets());  // patch inverses
 // z = sum_p R_p^T A_p^-1 R_p r
 void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets& ps = PatchSets());
+// the same for s = r - alpha v of a BiCGStab solve, alpha from nb <= 256 partials of (r^, v)
+void launch_patch_apply_s(cmg_ctx* c, const BicgVec& k, const double* part, int nb, double* z, const PatchSets& ps);
+// A x = b, right preconditioned with the context's preconditioner (built by the caller);
+// zero_guess: x starts at zero whatever it holds
+int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero_guess, double rtol, int maxit,
+             cmg_solve_stats* st);
 }  // namespace cmg

@@ -21,6 +21,7 @@
 #include <cstring>
 #include <vector>
 
+#include "bicgstab.h"
 #include "cmg_ctx.h"
 
 namespace cmg {
@@ -171,10 +172,11 @@ __device__ __forceinline__ void restrict_chunk(const CoarseGrid& g, int ch, cons
 }
 
 // y_p = A_p^{-1} r_p, one wave per patch, four patches per workgroup; the first g.n_rchunk
-// workgroups restrict r to the coarse grid instead
-template <typename IT>
-__global__ __launch_bounds__(256) void k_patch_apply(CoarseGrid g, const uint8_t* bcmask, double* rpart,
-                                                     int64_t set_rpart, int64_t P, const int32_t* pptr, const int32_t* pnodes,
+// workgroups restrict r to the coarse grid instead.  BICG: s = r - alpha v of a BiCGStab solve
+// (one set) in place of r, with alpha from the partials of (r^, v)
+template <typename IT, bool BICG>
+__global__ __launch_bounds__(256) void k_patch_apply(BicgVec kv, const double* apart, int na, CoarseGrid g,
+                                                     const uint8_t* bcmask, double* rpart, int64_t set_rpart, int64_t P, const int32_t* pptr, const int32_t* pnodes,
                                                      const int64_t* iptr, const IT* inv, const double* r,
                                                      double* y, int nd_max, int64_t set_inv, int64_t set_vec,
                                                      int64_t set_y, const int32_t* skip) {
@@ -184,7 +186,18 @@ __global__ __launch_bounds__(256) void k_patch_apply(CoarseGrid g, const uint8_t
     inv += set * set_inv;
     r += set * set_vec;
     y += set * set_y;
-    auto rhs = [&](int64_t i) { return r[i]; };
+    double alpha = 0.0;
+    if constexpr (BICG) {
+        __shared__ double sh4[4];
+        if (!bicg_alpha(kv, apart, na, sh4, alpha)) return;
+    }
+    const double* bv = kv.v;
+    auto rhs = [&](int64_t i) {
+        if constexpr (BICG)
+            return r[i] - alpha * bv[i];
+        else
+            return r[i];
+    };
     if ((int)blockIdx.x < g.n_rchunk) {
         restrict_chunk(g, (int)blockIdx.x, bcmask, rhs, rpart + set * set_rpart, lds);
         return;
@@ -359,7 +372,10 @@ void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps) {
     if (c->coarse) launch_coarse_setup(c, vals, ps);
 }
 
-void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets& ps) {
+namespace {
+
+void patch_apply(cmg_ctx* c, const BicgVec* kv, const double* apart, int na, const double* r, double* z,
+                 const PatchSets& ps) {
     const int ndm = c->sw_nd_max;
     const CoarseGrid g = c->coarse ? c->co : CoarseGrid();
     const CoarseBuf& cb = ps.coarse ? *ps.coarse : c->co_buf;
@@ -369,19 +385,34 @@ void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets&
     const size_t lds = (size_t)std::max(4 * ndm, 96) * sizeof(double);
     const void* inv = ps.inv ? ps.inv : c->sw_inv.p;
     double* y = ps.y ? ps.y : c->sw_y.as<double>();
-#define CMG_PAPPLY(IT)                                                                                              \
-    hipLaunchKernelGGL(k_patch_apply<IT>, grid, dim3(256), lds, c->stream, g, bc, cb.rpart.as<double>(), set_rpart, \
-                       c->sw_P, c->sw_pptr.as<int32_t>(), c->sw_pnodes.as<int32_t>(), c->sw_iptr.as<int64_t>(),     \
-                       (const IT*)inv, r, y, ndm, ps.set_inv, ps.set_vec, ps.set_y, ps.flags)
-    if (c->fp32)
-        CMG_PAPPLY(float);
-    else
-        CMG_PAPPLY(double);
+    const BicgVec k = kv ? *kv : BicgVec();
+#define CMG_PAPPLY(IT, BICG)                                                                                        \
+    hipLaunchKernelGGL((k_patch_apply<IT, BICG>), grid, dim3(256), lds, c->stream, k, apart, na, g, bc,             \
+                       cb.rpart.as<double>(), set_rpart, c->sw_P, c->sw_pptr.as<int32_t>(),                         \
+                       c->sw_pnodes.as<int32_t>(), c->sw_iptr.as<int64_t>(), (const IT*)inv, r, y, ndm, ps.set_inv, \
+                       ps.set_vec, ps.set_y, ps.flags)
+    if (c->fp32) {
+        if (kv) CMG_PAPPLY(float, true);
+        else CMG_PAPPLY(float, false);
+    } else {
+        if (kv) CMG_PAPPLY(double, true);
+        else CMG_PAPPLY(double, false);
+    }
 #undef CMG_PAPPLY
     if (c->coarse) launch_coarse_solve(c, ps);
     hipLaunchKernelGGL(k_patch_gather, dim3((unsigned)((c->N + 255) / 256), ps.S), dim3(256), 0, c->stream, g, bc,
                        cb.zc.as<double>(), c->N, c->sw_cptr.as<int32_t>(), c->sw_cpos.as<int32_t>(), y, z, ps.set_y,
                        ps.set_vec, ps.flags);
+}
+
+}  // namespace
+
+void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets& ps) {
+    patch_apply(c, nullptr, nullptr, 0, r, z, ps);
+}
+
+void launch_patch_apply_s(cmg_ctx* c, const BicgVec& k, const double* part, int nb, double* z, const PatchSets& ps) {
+    patch_apply(c, &k, part, nb, k.r, z, ps);
 }
 
 }  // namespace cmg

@@ -127,8 +127,8 @@ typedef struct cmg_options {
                                    element tangents written through LDS as contiguous 16-byte
                                    runs; 0 (default): 6 in FP64, 5 in mixed precision.  A context
                                    with a Land17 material always runs the shape of variant 6 */
-    int32_t krylov_method;      /* 0 GMRES(restart), 1 BiCGStab with device-side scalars and graph-replayed
-                                   iterations, 2 BiCGStab with host-side scalars (default); all right
+    int32_t krylov_method;      /* 0 GMRES(restart), 1 or 2 (default) BiCGStab with device-side scalars and
+                                   graph-replayed iterations (one solver, two accepted names); right
                                    preconditioned (see preconditioner) */
     double newton_atol;         /* Solver.Precision used as SNES abstol/rtol/stol (default 1e-8) */
     double newton_rtol;

@@ -1,0 +1,83 @@
+"""BiCGStab with device-side scalars (cmg_linear_solve): its iterates against the recurrence
+written out in numpy, and the true residual of converged solves, at the sizes where the
+product kernel's rows, partial sums and row groups end."""
+import numpy as np
+import pytest
+
+from cardiomechanics_amd import materials as MT
+from cardiomechanics_amd import mesh as M
+from cardiomechanics_amd.context import MechanicsContext
+
+pytestmark = pytest.mark.gpu
+
+
+def system(ctx, mesh):
+    """K + M / (beta dt^2) at the unloaded state, dt = 1 ms, in the context's value type"""
+    K, Mm = ctx.bsr(ctx.tangent(mesh.coords.ravel(), 0.0)), ctx.bsr(ctx.mass_matrix())
+    vals = np.ascontiguousarray((K.data.astype(np.float64) + Mm.data / 0.25e-6).reshape(-1), dtype=ctx.value_dtype)
+    A = ctx.bsr(vals)
+    A.data = A.data.astype(np.float64)
+    return vals, A.tocsr()
+
+
+def bicgstab(A, dinv, b, x, its):
+    """van der Vorst 1992 with right block Jacobi, r^ = r0"""
+    def pre(v):
+        return np.einsum("nij,nj->ni", dinv, v.reshape(-1, 3)).ravel()
+    r = b - A @ x
+    rh, p, rho = r.copy(), r.copy(), r @ r
+    for _ in range(its):
+        ph = pre(p)
+        v = A @ ph
+        alpha = rho / (rh @ v)
+        s = r - alpha * v
+        sh = pre(s)
+        t = A @ sh
+        om = (t @ s) / (t @ t)
+        x = x + alpha * ph + om * sh
+        r = s - om * t
+        rho, old = rh @ r, rho
+        p = r + rho / old * (alpha / om) * (p - om * v)
+    return x
+
+
+# nodes: 8, 27, 64, 343, and more than 256 partials of a product (a workgroup takes 8 or 16
+# rows): 3,375 nodes of T10, 8,000 of T4
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("order,n", [(4, 1), (10, 1), (4, 3), (10, 3), (10, 7), (4, 19)])
+def test_iterates_match_recurrence(order, n, precision):
+    """Four iterations from a guess.  Both sides round at 1e-16 per operation and the
+    recurrence amplifies that by the ratios rho / (r^, v), far below 1e7 in four iterations."""
+    mesh = M.cube_mesh(n, order=order)
+    rng = np.random.default_rng(5)
+    with MechanicsContext(mesh, [MT.cube_guccione()], preconditioner=1, precision=precision, krylov_maxit=4) as ctx:
+        vals, A = system(ctx, mesh)
+        b, x0 = rng.normal(size=ctx.n_dofs), 1e-9 * rng.normal(size=ctx.n_dofs)
+        x, st = ctx.linear_solve(vals, b, x0=x0, rtol=1e-15)
+        again, _ = ctx.linear_solve(vals, b, x0=x0, rtol=1e-15)
+    D = A.tobsr((3, 3))
+    diag = np.array([D.data[D.indptr[r]:D.indptr[r + 1]][D.indices[D.indptr[r]:D.indptr[r + 1]] == r][0]
+                     for r in range(len(D.indptr) - 1)])
+    ref = bicgstab(A, np.linalg.inv(diag), b, x0, 4)
+    assert st.iterations == 4 and not st.converged
+    assert x.tobytes() == again.tobytes()
+    assert np.linalg.norm(x - ref) <= 1e-9 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("pc", [1, 2], ids=["block_jacobi", "schwarz"])
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("size", [700, 50_000], ids=["one_row_group", "four_row_groups"])
+def test_true_residual_of_converged_solve(size, precision, pc):
+    """50,000 elements have more than 65,536 nodes, where a workgroup takes four row groups."""
+    mesh = M.lv_mesh(size)
+    rng = np.random.default_rng(6)
+    with MechanicsContext(mesh, [MT.lv_holzapfel()], preconditioner=pc, precision=precision) as ctx:
+        assert size < 50_000 or ctx.n_dofs > 3 * 65_536
+        vals, A = system(ctx, mesh)
+        b = A @ rng.normal(size=ctx.n_dofs)
+        x, st = ctx.linear_solve(vals, b, rtol=1e-6)
+        z, sz = ctx.linear_solve(vals, np.zeros_like(b), x0=np.zeros_like(b), rtol=1e-6)
+    assert st.converged and st.iterations > 0
+    # the solver's own last residual is b - A x in double: rounding aside, the same number
+    assert np.linalg.norm(b - A @ x) <= 1.000001e-6 * np.linalg.norm(b)
+    assert sz.converged and sz.iterations == 0 and not z.any()
