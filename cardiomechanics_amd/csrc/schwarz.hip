@@ -11,8 +11,9 @@
 //
 // Device work per tangent: one wave per patch gathers A_p from the block values into
 // LDS and inverts it by Gauss-Jordan elimination with partial pivoting (FP64), storing
-// the inverse column-major (FP64, or FP32 in mixed precision).  Per application: one
-// wave per patch forms y_p = A_p^{-1} r_p (lane i owns row i: coalesced column reads),
+// the inverse in groups of kGroup columns (FP64, or FP32 in mixed precision): a lane's
+// entries of one row and group are 16 consecutive bytes.  Per application: one
+// wave per patch forms y_p = A_p^{-1} r_p (lane i owns row i: coalesced group reads),
 // then every node sums its one or two patch results in patch order (deterministic,
 // no atomics) and the coarse-grid correction (coarse.hip).
 #include <algorithm>
@@ -28,6 +29,8 @@ namespace cmg {
 namespace {
 
 constexpr int kWave = 64;
+template <typename IT>
+constexpr int kGroup = 16 / sizeof(IT);   // columns of an inverse stored together: [group][row][kGroup]
 
 // A_p^{-1} of the patches order[0, n), one wave per patch.  Dynamic LDS: nd_cap^2 +
 // nd_cap doubles + nd_cap ints for the class's largest patch.  Gauss-Jordan with
@@ -133,8 +136,10 @@ __global__ __launch_bounds__(kWave) void k_patch_setup(int64_t n, const int32_t*
         __syncthreads();
     }
     IT* out = inv + iptr[p];
-    for (int j = 0; j < nd; j++)   // column-major: out[j nd + i] = Ainv[i][j]
-        for (int i = lane; i < nd; i += kWave) out[(int64_t)j * nd + i] = (IT)A[i * nd + j];
+    constexpr int G = kGroup<IT>;
+    for (int j = 0; j < (nd + G - 1) / G * G; j++)   // columns past nd are zero
+        for (int i = lane; i < nd; i += kWave)
+            out[((int64_t)(j / G) * nd + i) * G + j % G] = j < nd ? (IT)A[i * nd + j] : (IT)0;
 }
 
 // restriction partials of one chunk of fine nodes (all of one grid cell): [corner][component],
@@ -159,24 +164,45 @@ __device__ __forceinline__ void restrict_chunk(const CoarseGrid& g, int ch, cons
             for (int i = 0; i < 3; i++) s[3 * a + i] += w * v[i];
         }
     }
+    // 24 sums over the wave: a halving exchange leaves each lane three of them in 21 exchanges
+    // (x, y and z of corner lane / 8), three more steps finish them; one by one they are 144
     const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
 #pragma unroll
-    for (int q = 0; q < 24; q++) {
+    for (int o = 32, h = 12; o >= 8; o >>= 1, h /= 2) {
+        const bool up = (lane & o) != 0;
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s[q] += __shfl_xor(s[q], o, 64);
-        if (lane == 0) sh[24 * w + q] = s[q];
+        for (int q = 0; q < h; q++) {
+            const double give = up ? s[q] : s[h + q], keep = up ? s[h + q] : s[q];
+            s[q] = keep + __shfl_xor(give, o, 64);
+        }
     }
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1)
+#pragma unroll
+        for (int i = 0; i < 3; i++) s[i] += __shfl_xor(s[i], o, 64);
+    if (lane % 8 == 0)
+#pragma unroll
+        for (int i = 0; i < 3; i++) sh[24 * w + 3 * (lane / 8) + i] = s[i];
     __syncthreads();
     if (threadIdx.x < 24)
-        out[3 * (int64_t)g.rslot[8 * ch + threadIdx.x / 3] + threadIdx.x % 3] = sh[threadIdx.x] + sh[24 + threadIdx.x] + sh[48 + threadIdx.x] + sh[72 + threadIdx.x];
+        out[3 * (int64_t)g.rslot[8 * ch + threadIdx.x / 3] + threadIdx.x % 3] =
+            sh[threadIdx.x] + sh[24 + threadIdx.x] + sh[48 + threadIdx.x] + sh[72 + threadIdx.x];
 }
 
-// y_p = A_p^{-1} r_p, one wave per patch, four patches per workgroup; the first g.n_rchunk
-// workgroups restrict r to the coarse grid instead.  BICG: s = r - alpha v of a BiCGStab solve
+// y_p = A_p^{-1} r_p, one wave per patch, four patches per workgroup; bound by the inverses
+// (548 MB on the 200k-element LV) or, on small meshes, by its chain of dependent loads.  Loads
+// return in order, so they are issued as they are needed: the patch's nodes, the first
+// U groups of the lane's row of the inverse (all of an average patch), the right-hand side
+// at the nodes, and only then alpha is formed.  One column
+// per load, requested after the right-hand side and behind alpha, took (us, plain / BICG): 200k
+// LV 119 / 125 now 105 / 103, FP32 78 / 93 now 58 / 60, 20k LV 14.2 / 17.4 now 12.3 / 14.9,
+// 1,296-element cube 8.0 / 9.0 now 4.1 / 4.8.
+// The first g.n_rchunk workgroups restrict r to the coarse grid instead.  BICG: s = r - alpha v of a BiCGStab solve
 // (one set) in place of r, with alpha from the partials of (r^, v)
 template <typename IT, bool BICG>
 __global__ __launch_bounds__(256) void k_patch_apply(BicgVec kv, const double* apart, int na, CoarseGrid g,
-                                                     const uint8_t* bcmask, double* rpart, int64_t set_rpart, int64_t P, const int32_t* pptr, const int32_t* pnodes,
+                                                     const uint8_t* bcmask, double* rpart, int64_t set_rpart,
+                                                     int64_t P, const int32_t* pptr, const int32_t* pnodes,
                                                      const int64_t* iptr, const IT* inv, const double* r,
                                                      double* y, int nd_max, int64_t set_inv, int64_t set_vec,
                                                      int64_t set_y, const int32_t* skip) {
@@ -186,37 +212,73 @@ __global__ __launch_bounds__(256) void k_patch_apply(BicgVec kv, const double* a
     inv += set * set_inv;
     r += set * set_vec;
     y += set * set_y;
-    double alpha = 0.0;
-    if constexpr (BICG) {
-        __shared__ double sh4[4];
-        if (!bicg_alpha(kv, apart, na, sh4, alpha)) return;
-    }
+    __shared__ double sh4[4];
     const double* bv = kv.v;
-    auto rhs = [&](int64_t i) {
-        if constexpr (BICG)
-            return r[i] - alpha * bv[i];
-        else
-            return r[i];
-    };
     if ((int)blockIdx.x < g.n_rchunk) {
+        double alpha = 0.0;
+        if (BICG && !bicg_alpha(kv, apart, na, sh4, alpha)) return;
+        auto rhs = [&](int64_t i) { return BICG ? r[i] - alpha * bv[i] : r[i]; };
         restrict_chunk(g, (int)blockIdx.x, bcmask, rhs, rpart + set * set_rpart, lds);
         return;
     }
-    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    // the wave's number as a scalar: the patch's sizes and offsets become scalar loads and branches
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const int64_t p = ((int64_t)blockIdx.x - g.n_rchunk) * 4 + w;
+    constexpr int G = kGroup<IT>;
+    typedef IT VG __attribute__((ext_vector_type(G)));
+    constexpr int U = sizeof(IT) == 8 ? 20 : 12;   // groups requested ahead
     double* rp = lds + (size_t)w * nd_max;
-    const bool valid = p < P;
-    const int p0 = valid ? pptr[p] : 0;
-    const int nd = valid ? 3 * (pptr[p + 1] - p0) : 0;
-    for (int l = lane; l < nd; l += kWave) rp[l] = rhs(3 * (int64_t)pnodes[p0 + l / 3] + l % 3);
-    __syncthreads();
-    if (!valid) return;
-    const IT* a = inv + iptr[p];
+    int p0 = 0, nd = 0;
+    const VG* a = nullptr;
+    if (p < P) {
+        p0 = pptr[p];
+        nd = 3 * (pptr[p + 1] - p0);
+        a = reinterpret_cast<const VG*>(inv + iptr[p]);
+    }
+    const int ng = (nd + G - 1) / G;
+    VG pre[U];
+    double rv = 0.0, vv = 0.0;
+    if (lane < nd) {
+        const int64_t at = 3 * (int64_t)pnodes[p0 + lane / 3] + lane % 3;
+#pragma unroll
+        for (int u = 0; u < U; u++) pre[u] = a[(u < ng ? u : 0) * nd + lane];
+        rv = r[at];
+        if (BICG) vv = bv[at];
+    }
+    double alpha = 0.0;
+    if (BICG && !bicg_alpha(kv, apart, na, sh4, alpha)) return;
+    if (nd == 0) return;   // past the last patch
+    auto entry = [&](int l) {   // of a patch of more than 64 DOFs
+        const int64_t at = 3 * (int64_t)pnodes[p0 + l / 3] + l % 3;
+        return BICG ? r[at] - alpha * bv[at] : r[at];
+    };
+    if (lane < ng * G) rp[lane] = BICG ? rv - alpha * vv : rv;
+    for (int l = lane + kWave; l < ng * G; l += kWave) rp[l] = l < nd ? entry(l) : 0.0;
+    __builtin_amdgcn_wave_barrier();   // rp belongs to this wave; its LDS operations keep their order
     double* yo = y + 3 * (int64_t)p0;
-    for (int i = lane; i < nd; i += kWave) {
+    if (lane < nd) {
         double acc = 0.0;
-        for (int j = 0; j < nd; j++) acc += (double)a[(int64_t)j * nd + i] * rp[j];
-        yo[i] = acc;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (u < ng) {
+#pragma unroll
+                for (int q = 0; q < G; q++) acc += (double)pre[u][q] * rp[G * u + q];
+            }
+        for (int gr = U; gr < ng; gr++) {
+            const VG v = a[gr * nd + lane];
+#pragma unroll
+            for (int q = 0; q < G; q++) acc += (double)v[q] * rp[G * gr + q];
+        }
+        yo[lane] = acc;
+    }
+    for (int i = lane + kWave; i < nd; i += kWave) {   // the few patches of more than 64 DOFs
+        double s = 0.0;
+        for (int gr = 0; gr < ng; gr++) {
+            const VG v = a[(int64_t)gr * nd + i];
+#pragma unroll
+            for (int q = 0; q < G; q++) s += (double)v[q] * rp[G * gr + q];
+        }
+        yo[i] = s;
     }
 }
 
@@ -317,7 +379,8 @@ int build_vertex_patches(cmg_ctx* c, const int32_t* elements) {
                 slots.push_back((f != e && *f == q[j]) ? (int32_t)(c->h_rowptr[q[i]] + (f - b)) : -1);
             }
         sptr[p + 1] = (int64_t)slots.size();
-        iptr[p + 1] = iptr[p] + (int64_t)9 * np * np;
+        const int gc = c->fp32 ? kGroup<float> : kGroup<double>;
+        iptr[p + 1] = iptr[p] + (int64_t)(3 * np) * ((3 * np + gc - 1) / gc * gc);
     }
     // node -> positions of its rows in y (y rows follow pnodes), in patch order
     std::vector<int32_t> cnt(N + 1, 0);
@@ -376,7 +439,7 @@ namespace {
 
 void patch_apply(cmg_ctx* c, const BicgVec* kv, const double* apart, int na, const double* r, double* z,
                  const PatchSets& ps) {
-    const int ndm = c->sw_nd_max;
+    const int ndm = (c->sw_nd_max + 3) / 4 * 4;   // whole groups
     const CoarseGrid g = c->coarse ? c->co : CoarseGrid();
     const CoarseBuf& cb = ps.coarse ? *ps.coarse : c->co_buf;
     const int64_t set_rpart = (int64_t)g.n_rchunk * 24;
