@@ -33,6 +33,9 @@ struct DevBuf {
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
+// size classes of the Schwarz patches: up to 24, 30, 36, 42, 48, 54, 60 DOFs, and larger
+constexpr int kPatchClasses = 8;
+
 // background grid of the coarse correction (coarse.hip) and the fine nodes' place in it
 struct CoarseGrid {
     int nodes = 0, ld = 0;              // grid nodes, leading dimension of A_c (3 nodes, padded)
@@ -159,12 +162,10 @@ struct cmg_ctx {
     int64_t sw_P = 0;
     int sw_nd_max = 0;
     cmg::DevBuf sw_pptr, sw_pnodes, sw_sptr, sw_slots, sw_iptr, sw_cptr, sw_cpos, sw_inv, sw_y;
-    // patches by size class for the setup launches: sw_order[0, sw_n_small) have at most
-    // sw_nd_small DOFs, the rest up to sw_nd_max
+    // patches by size class for the setup launches: class k is sw_order[sw_cls[k], sw_cls[k + 1])
     cmg::DevBuf sw_order;
+    int64_t sw_cls[cmg::kPatchClasses + 1] = {};
     bool precond_built = false;   // the preconditioner holds a factorisation of this Newton solve
-    int64_t sw_n_small = 0;
-    int sw_nd_small = 0;
     int64_t sw_inv_len = 0, sw_y_len = 0;   // inverse values and patch-vector rows of all patches
     // coarse-grid correction of the Schwarz preconditioner (coarse.hip)
     bool coarse = false;

@@ -32,8 +32,8 @@ constexpr int kWave = 64;
 template <typename IT>
 constexpr int kGroup = 16 / sizeof(IT);   // columns of an inverse stored together: [group][row][kGroup]
 
-// A_p^{-1} of the patches order[0, n), one wave per patch.  Dynamic LDS: nd_cap^2 +
-// nd_cap doubles + nd_cap ints for the class's largest patch.  Gauss-Jordan with
+// A_p^{-1} of the patches order[0, n) that k_patch_invert has no registers for, one wave per
+// patch.  Dynamic LDS: nd_cap^2 + nd_cap doubles + nd_cap ints for the largest patch.  Gauss-Jordan with
 // partial pivoting; in the elimination each lane owns columns j = lane, lane + 64 and
 // walks the rows, so no index is divided and the pivot row stays in registers.
 template <typename VT, typename IT>
@@ -189,6 +189,85 @@ __device__ __forceinline__ void restrict_chunk(const CoarseGrid& g, int ch, cons
             sh[threadIdx.x] + sh[24 + threadIdx.x] + sh[48 + threadIdx.x] + sh[72 + threadIdx.x];
 }
 
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// A_p^{-1} of patches of at most ND DOFs, in registers: lane i holds row i.  Gauss-Jordan with
+// partial pivoting, rows left in place: step k picks the free lane with the largest entry of
+// column k (by the upper 32 bits of its magnitude, the lowest lane among equals), broadcasts
+// its row through scalar registers and subtracts multiples of it from every other row.  The
+// pivot row is scaled at the end instead, so one fused multiply-add per entry and step
+// remains.  Columns rotate by one register per step, which keeps every register index fixed
+// in a loop that is not unrolled.  Bound by the vector ALUs: two lane reads and one
+// multiply-add per entry (all
+// patches of a setup: 200k LV 5.3 ms in LDS, 1.2 ms; 20k LV 1.0 / 0.54 ms; eight sets of 5k
+// 0.83 / 0.30 ms; cube 0.26 / 0.14 ms).
+template <typename VT, typename IT, int ND>
+__global__ __launch_bounds__(256) void k_patch_invert(int64_t n, const int32_t* order, const int32_t* pptr,
+                                                      const int64_t* sptr, const int32_t* slots, const int64_t* iptr,
+                                                      const VT* vals, IT* inv, int64_t set_vals, int64_t set_inv,
+                                                      const int32_t* active) {
+    const int64_t set = blockIdx.y;
+    if (active && !active[set]) return;
+    const int64_t idx = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;
+    if (idx >= n) return;   // whole waves
+    vals += set * set_vals;
+    inv += set * set_inv;
+    const int64_t p = order[idx];
+    const int lane = threadIdx.x % kWave;
+    const int np = __builtin_amdgcn_readfirstlane(pptr[p + 1] - pptr[p]), nd = 3 * np;
+    const int32_t* sl = slots + sptr[p];
+    const int bi = lane / 3, ci = lane - 3 * bi;
+    double a[ND];
+#pragma unroll
+    for (int bj = 0; bj < ND / 3; bj++) {
+        if (bj < np) {
+            const int s = lane < nd ? sl[bi * np + bj] : -1;
+#pragma unroll
+            for (int c = 0; c < 3; c++) a[3 * bj + c] = s >= 0 ? (double)vals[9 * (int64_t)s + 3 * ci + c] : 0.0;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 3; c++) a[3 * bj + c] = 3 * bj + c == lane ? 1.0 : 0.0;   // identity padding
+        }
+    }
+    bool used = lane >= ND;
+    int row = -1, perm = 0;      // the row of the inverse this lane ends with; lane k: the pivot lane of step k
+    double scale = 1.0;
+#pragma unroll 1
+    for (int k = 0; k < ND; k++) {
+        const unsigned key = used ? 0u : ((unsigned)(__double_as_longlong(a[0]) >> 32) & 0x7fffffffu) + 1u;
+        unsigned best = key;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) best = max(best, (unsigned)__shfl_xor((int)best, o));
+        const int piv_lane = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(key == best && !used)) - 1);
+        const double ip = 1.0 / read_lane(a[0], piv_lane);
+        const bool mine = lane == piv_lane;
+        const double m = mine ? 0.0 : a[0] * ip;
+        if (mine) {
+            used = true;
+            row = k;
+            scale = ip;
+        }
+        if (lane == k) perm = piv_lane;
+#pragma unroll
+        for (int j = 1; j < ND; j++) a[j - 1] = fma(-m, read_lane(a[j], piv_lane), a[j]);
+        a[ND - 1] = mine ? 1.0 : -m;
+    }
+    constexpr int G = kGroup<IT>;
+    IT* out = inv + iptr[p];
+#pragma unroll
+    for (int j = 0; j < ND; j++) {
+        const int c = __builtin_amdgcn_readlane(perm, j);
+        if (j < nd && c < nd && row >= 0 && row < nd) out[((int64_t)(c / G) * nd + row) * G + c % G] = (IT)(a[j] * scale);
+    }
+    for (int c = nd; c < (nd + G - 1) / G * G; c++)   // columns past nd are zero
+        if (lane < nd) out[((int64_t)(c / G) * nd + lane) * G + c % G] = (IT)0;
+}
+
 // y_p = A_p^{-1} r_p, one wave per patch, four patches per workgroup; bound by the inverses
 // (548 MB on the 200k-element LV) or, on small meshes, by its chain of dependent loads.  Loads
 // return in order, so they are issued as they are needed: the patch's nodes, the first
@@ -284,9 +363,9 @@ __global__ __launch_bounds__(256) void k_patch_apply(BicgVec kv, const double* a
 
 // z[3n + c] = sum over the patches holding node n of their y rows, in patch order, plus the
 // coarse correction at the node (g.nodes > 0)
-__global__ __launch_bounds__(256) void k_patch_gather(CoarseGrid g, const uint8_t* bcmask, const double* zc, int64_t N, const int32_t* cptr, const int32_t* cpos,
-                                                      const double* y, double* z, int64_t set_y, int64_t set_vec,
-                                                      const int32_t* skip) {
+__global__ __launch_bounds__(256) void k_patch_gather(CoarseGrid g, const uint8_t* bcmask, const double* zc, int64_t N,
+                                                      const int32_t* cptr, const int32_t* cpos, const double* y,
+                                                      double* z, int64_t set_y, int64_t set_vec, const int32_t* skip) {
     const int64_t set = blockIdx.y;
     if (skip && skip[set]) return;
     y += set * set_y;
@@ -353,16 +432,18 @@ int build_vertex_patches(cmg_ctx* c, const int32_t* elements) {
         np_max = std::max(np_max, (int)q.size());
     }
     if (3 * np_max > kMaxPatchDofs) return CMG_SUCCESS;   // stays with block Jacobi
-    // setup launches by size class: patches of at most kSmallPatchDofs DOFs (most of
-    // them) with that much LDS per wave, the rest with room for the largest
-    constexpr int kSmallPatchDofs = 48;
+    // setup launches by size class: up to 24, 30, ... 60 DOFs in registers, the rest in LDS
     std::vector<int32_t> order;
     order.reserve(P);
-    for (int64_t p = 0; p < P; p++)
-        if (3 * (int)patch[p].size() <= kSmallPatchDofs) order.push_back((int32_t)p);
-    const int64_t n_small = (int64_t)order.size();
-    for (int64_t p = 0; p < P; p++)
-        if (3 * (int)patch[p].size() > kSmallPatchDofs) order.push_back((int32_t)p);
+    c->sw_cls[0] = 0;
+    for (int k = 0; k < kPatchClasses; k++) {
+        for (int64_t p = 0; p < P; p++) {
+            const int nd = 3 * (int)patch[p].size();
+            const int cls = nd <= 24 ? 0 : std::min(kPatchClasses - 1, (nd - 24 + 5) / 6);
+            if (cls == k) order.push_back((int32_t)p);
+        }
+        c->sw_cls[k + 1] = (int64_t)order.size();
+    }
     std::vector<int32_t> pptr(P + 1, 0), pnodes;
     std::vector<int64_t> sptr(P + 1, 0), iptr(P + 1, 0);
     std::vector<int32_t> slots;
@@ -404,34 +485,54 @@ int build_vertex_patches(cmg_ctx* c, const int32_t* elements) {
     CMG_HIP_CHECK(hipStreamSynchronize(s));
     c->sw_P = P;
     c->sw_nd_max = 3 * np_max;
-    c->sw_n_small = n_small;
-    c->sw_nd_small = std::min(kSmallPatchDofs, 3 * np_max);
     c->sw_inv_len = iptr[P];
     c->sw_y_len = 3 * (int64_t)pnodes.size();
     c->schwarz = true;
     return CMG_SUCCESS;
 }
 
-void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps) {
-    const int64_t cls_n[2] = {c->sw_n_small, c->sw_P - c->sw_n_small};
-    const int cls_nd[2] = {c->sw_nd_small, c->sw_nd_max};
-    void* inv = ps.inv ? ps.inv : c->sw_inv.p;
-    for (int k = 0; k < 2; k++) {
-        if (cls_n[k] == 0) continue;
-        const int nd = cls_nd[k];
-        const size_t lds = (size_t)(nd * nd + nd) * sizeof(double) + (size_t)nd * sizeof(int);
-        const int32_t* order = c->sw_order.as<int32_t>() + (k ? c->sw_n_small : 0);
-        const dim3 grid((unsigned)cls_n[k], ps.S);
-#define CMG_PSETUP(VT, IT)                                                                                           \
-    hipLaunchKernelGGL((k_patch_setup<VT, IT>), grid, dim3(kWave), lds, c->stream, cls_n[k], order,                 \
-                       c->sw_pptr.as<int32_t>(), c->sw_sptr.as<int64_t>(), c->sw_slots.as<int32_t>(),              \
-                       c->sw_iptr.as<int64_t>(), (const VT*)vals, (IT*)inv, nd, ps.set_vals, ps.set_inv, ps.flags)
-        if (c->fp32)
-            CMG_PSETUP(float, float);
-        else
-            CMG_PSETUP(double, double);
-#undef CMG_PSETUP
+namespace {
+
+template <typename VT, typename IT>
+void patch_setup(cmg_ctx* c, const VT* vals, IT* inv, const PatchSets& ps) {
+    for (int k = 0; k < kPatchClasses; k++) {
+        const int64_t n = c->sw_cls[k + 1] - c->sw_cls[k];
+        if (n == 0) continue;
+        const int32_t* order = c->sw_order.as<int32_t>() + c->sw_cls[k];
+        const int32_t* pptr = c->sw_pptr.as<int32_t>();
+        const int64_t *sptr = c->sw_sptr.as<int64_t>(), *iptr = c->sw_iptr.as<int64_t>();
+        const int32_t* slots = c->sw_slots.as<int32_t>();
+        const dim3 grid((unsigned)((n + 3) / 4), ps.S);
+#define CMG_PINV(ND)                                                                                                \
+    hipLaunchKernelGGL((k_patch_invert<VT, IT, ND>), grid, dim3(256), 0, c->stream, n, order, pptr, sptr, slots, iptr, \
+                       vals, inv, ps.set_vals, ps.set_inv, ps.flags)
+        switch (k) {
+        case 0: CMG_PINV(24); break;
+        case 1: CMG_PINV(30); break;
+        case 2: CMG_PINV(36); break;
+        case 3: CMG_PINV(42); break;
+        case 4: CMG_PINV(48); break;
+        case 5: CMG_PINV(54); break;
+        case 6: CMG_PINV(60); break;
+        default: {
+            const int nd = c->sw_nd_max;
+            const size_t lds = (size_t)(nd * nd + nd) * sizeof(double) + (size_t)nd * sizeof(int);
+            hipLaunchKernelGGL((k_patch_setup<VT, IT>), dim3((unsigned)n, ps.S), dim3(kWave), lds, c->stream, n, order,
+                               pptr, sptr, slots, iptr, vals, inv, nd, ps.set_vals, ps.set_inv, ps.flags);
+        }
+        }
+#undef CMG_PINV
     }
+}
+
+}  // namespace
+
+void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps) {
+    void* inv = ps.inv ? ps.inv : c->sw_inv.p;
+    if (c->fp32)
+        patch_setup(c, (const float*)vals, (float*)inv, ps);
+    else
+        patch_setup(c, (const double*)vals, (double*)inv, ps);
     if (c->coarse) launch_coarse_setup(c, vals, ps);
 }
 

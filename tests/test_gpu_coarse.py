@@ -6,6 +6,7 @@ pivot changes the preconditioner and with it the count."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
+from scipy.spatial import ConvexHull
 
 from cardiomechanics_amd import materials as MT
 from cardiomechanics_amd import mesh as M
@@ -69,6 +70,13 @@ def preconditioner(mesh, K):
     free = np.ones(3 * len(X))
     for c in range(3):
         free[c::3][(mesh.bc >> c) & 1 == 1] = 0.0
+    if len(ps) // 4 < 8:   # too few patches for a grid
+        def apply(r):
+            z = np.zeros_like(r)
+            for d, Ap in inverses:
+                z[d] += Ap @ r[d]
+            return z
+        return apply, 0
     P = sp.diags(free) @ sp.kron(background_grid(X, el, min(340, len(ps) // 4)), sp.eye(3)).tocsr()
     Ac = (P.T @ K @ P).toarray()
     keep = np.diag(Ac) > 0
@@ -101,12 +109,32 @@ def gmres_count(K, pre, b, rtol, m=400):
     return m
 
 
+def star(points):
+    """tetrahedra between the origin and the hull of `points` points on a sphere: the origin's
+    patch has 3 (points + 1) components"""
+    k = np.arange(points) + 0.5
+    z, phi = 1 - 2 * k / points, np.pi * (1 + 5 ** 0.5) * k
+    v = 0.01 * np.stack([np.sqrt(1 - z * z) * np.cos(phi), np.sqrt(1 - z * z) * np.sin(phi), z], 1)
+    tets = np.concatenate([ConvexHull(v).simplices, np.full((2 * points - 4, 1), points)], 1)
+    X = np.concatenate([v, np.zeros((1, 3))])
+    coords, el, _ = M.t4_to_t10(X, M.orient_t4(X, tets))
+    E = len(el)
+    return M.Mesh(coords=coords, elements=el.astype(np.int32), bases=np.tile(np.eye(3), (E, 5, 1, 1)),
+                  bc=np.zeros(len(coords), np.uint8), material=np.zeros(E, np.int32), activation=np.zeros(E),
+                  name=f"lv-like star {points}")
+
+
 MESHES = {   # grid nodes: 8 (one padded panel), 27, a ventricle with constrained base, two panels and more
     "cube3": lambda: (M.cube_mesh(3), MT.cube_guccione()),
     "cube4": lambda: (M.cube_mesh(4), MT.cube_guccione()),
     "cube5": lambda: (M.cube_mesh(5), MT.cube_guccione()),
     "lv_900": lambda: (M.lv_mesh(900), MT.lv_holzapfel()),
     "lv_2500": lambda: (M.lv_mesh(2500), MT.lv_holzapfel()),
+    # largest patch 24 to 72 components, the most that patches may have: the register inversion ends its
+    # classes at 24, 30, ..
+    # 60, and an application's lanes at 64
+    **{f"star_{n}": (lambda n=n: (star(n), MT.lv_holzapfel()))
+       for n in (7, 8, 9, 11, 12, 13, 15, 16, 17, 18, 19, 20, 21, 23)},
 }
 
 
