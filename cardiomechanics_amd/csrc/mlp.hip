@@ -2,8 +2,8 @@
 // 8 -> H -> H -> 3 (tanh hidden layers) that maps nodal features of the next
 // Newmark step (the two previous increments, the pressure rate and the activation
 // phase) to that step's displacement increment.  Hand-written gfx950 kernels for
-// inference, the backward pass (activation gradients and weight-gradient
-// reductions, two-stage and in a fixed order) and Adam.  The step only uses the
+// inference, the training pass (forward, backward and all weight gradients in one
+// kernel, partial sums added in a fixed order) and Adam.  The step only uses the
 // proposed guess when its residual is below the predictor's (the predictor is both
 // the fallback and the yardstick).
 //
@@ -25,10 +25,10 @@ namespace {
 constexpr int kH = 128;         // hidden width of the kernels
 constexpr int kIn = 8;
 constexpr int kOut = 3;
-constexpr int kTile = 64;       // rows per tile
 constexpr int kThr = 256;       // threads per workgroup
-constexpr int kPad = kH + 1;    // LDS row pitch (bank-conflict-free column walks)
-constexpr int kGradBlocks = 128;
+constexpr int kWaveRows = 16;   // rows of one wave's tile
+constexpr int kTile = 64;       // rows of a training workgroup's tile (four waves)
+constexpr int kTrainBlocks = 256;   // partial gradients: one training workgroup per CU
 
 constexpr int64_t n_weights() { return kIn * kH + kH + kH * kH + kH + kH * kOut + kOut; }
 constexpr int64_t off_b1 = kIn * kH;
@@ -37,357 +37,477 @@ constexpr int64_t off_b2 = off_W2 + kH * kH;
 constexpr int64_t off_W3 = off_b2 + kH;
 constexpr int64_t off_b3 = off_W3 + kH * kOut;
 
-__device__ __forceinline__ float bf16_round(float x) {
-    // round to nearest even at bfloat16 precision (finite inputs)
-    uint32_t u = __float_as_uint(x);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return __uint_as_float(u & 0xffff0000u);
-}
-
-// ---------------------------------------------------------------------------
-// forward (FP32): grid-stride over 64-row tiles; W2 stays in LDS for all tiles of a
-// block.  Thread t owns rows 4*(t/16)..+4 and hidden columns 8*(t%16)..+8.
-// store_act: write the hidden activations A1, A2 [rows][H] (training).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThr) void k_mlp_forward(const float* __restrict__ w, const float* __restrict__ X,
-                                                      int64_t rows, float* __restrict__ Y, float* __restrict__ A1g,
-                                                      float* __restrict__ A2g) {
-    __shared__ float sW2[kH * kH];
-    __shared__ float sW1[kIn * kH];
-    __shared__ float sb1[kH], sb2[kH];
-    __shared__ float sW3[kH * kOut];
-    __shared__ float sb3[kOut];
-    __shared__ float sA[kTile * kPad];
-    const int t = threadIdx.x;
-    for (int i = t; i < kH * kH; i += kThr) sW2[i] = w[off_W2 + i];
-    for (int i = t; i < kIn * kH; i += kThr) sW1[i] = w[i];
-    for (int i = t; i < kH * kOut; i += kThr) sW3[i] = w[off_W3 + i];
-    if (t < kH) {
-        sb1[t] = w[off_b1 + t];
-        sb2[t] = w[off_b2 + t];
-    }
-    if (t < kOut) sb3[t] = w[off_b3 + t];
-    __syncthreads();
-    const int rg = t / 16, cg = t % 16;
-    const int64_t ntiles = (rows + kTile - 1) / kTile;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t r0 = tile * kTile;
-        // ---- layer 1 ----
-        float acc[4][8];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int64_t r = r0 + rg * 4 + i;
-            float x[kIn];
-#pragma unroll
-            for (int k = 0; k < kIn; k++) x[k] = (r < rows) ? X[r * kIn + k] : 0.f;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int c = cg * 8 + j;
-                float s = sb1[c];
-#pragma unroll
-                for (int k = 0; k < kIn; k++) s += x[k] * sW1[k * kH + c];
-                acc[i][j] = tanhf(s);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int64_t r = r0 + rg * 4 + i;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                sA[(rg * 4 + i) * kPad + cg * 8 + j] = acc[i][j];
-                if (A1g && r < rows) A1g[r * kH + cg * 8 + j] = acc[i][j];
-            }
-        }
-        __syncthreads();
-        // ---- layer 2 ----
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) acc[i][j] = sb2[cg * 8 + j];
-        for (int k = 0; k < kH; k++) {
-            float a[4], b[8];
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = sA[(rg * 4 + i) * kPad + k];
-#pragma unroll
-            for (int j = 0; j < 8; j++) b[j] = sW2[k * kH + cg * 8 + j];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc[i][j] += a[i] * b[j];
-        }
-        __syncthreads();   // every thread is done reading A1 from LDS
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int64_t r = r0 + rg * 4 + i;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float h = tanhf(acc[i][j]);
-                sA[(rg * 4 + i) * kPad + cg * 8 + j] = h;
-                if (A2g && r < rows) A2g[r * kH + cg * 8 + j] = h;
-            }
-        }
-        __syncthreads();
-        // ---- layer 3: 64 rows x 3 outputs on threads 0..191 ----
-        if (t < kTile * kOut) {
-            const int rr = t / kOut, o = t % kOut;
-            const int64_t r = r0 + rr;
-            float s = sb3[o];
-            for (int k = 0; k < kH; k++) s += sA[rr * kPad + k] * sW3[k * kOut + o];
-            if (r < rows) Y[r * kOut + o] = s;
-        }
-        __syncthreads();   // sA is rewritten by the next tile
-    }
-}
-
-// ---------------------------------------------------------------------------
-// bfloat16 inference: the 128 x 128 layer on the matrix cores
-// (v_mfma_f32_16x16x16_bf16, FP32 accumulation), layers 1 and 3 in FP32 on the vector
-// ALUs; inputs, weights and both hidden activations rounded to bfloat16.  One wave per
-// 16 rows (four waves, 64 rows per tile).  Operand layout of the instruction (index
-// m % 4 is the item within a lane's four values):
-//   A[i][k] in lane i + 16 (k / 4),  B[k][j] in lane j + 16 (k / 4),  D[i][j] in lane j + 16 (i / 4).
-// A lane therefore computes its own layer-1 values straight into its A operands
-// (row i = lane % 16, columns 16 ks + 4 (lane / 16) + 0..3 for k-step ks), reads B from
-// W2 stored transposed in LDS (four consecutive k in 8 bytes), and ends with the
-// layer-2 outputs of rows 4 (lane / 16) + 0..3 and columns 16 nb + lane % 16, whose
-// layer-3 products are summed over the 16 lanes of a row group.
-// ---------------------------------------------------------------------------
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kW2tPitch = kH + 8;   // shorts per row of the transposed W2 (spreads the lanes over banks)
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ short bf16_bits(float x) {
-    uint32_t u = __float_as_uint(x);
-    u += 0x7fffu + ((u >> 16) & 1u);   // round to nearest even (finite inputs)
-    return (short)(u >> 16);
+// ---------------------------------------------------------------------------
+// All kernels hold activations transposed, H^T[c][row], in the output layout of the
+// 16x16 matrix instructions: lane 16 g + i has row i and columns 16 b + 4 g + s in
+// component s of register b.  Read as the second operand of the next product, that
+// register s of block b is one k-step over the columns 16 b + 4 g + s of the four lane
+// groups g, so the layers of a row follow each other in one wave's registers, and only
+// the weights come from LDS.  Operand layouts (i, j < 16):
+//   16x16x4 f32    A[i][k] lane i + 16 k,  B[k][j] lane j + 16 k
+//   16x16x16 bf16  A[i][k] lane i + 16 (k / 4), B alike, item k % 4
+//   16x16x32 bf16  A[i][k] lane i + 16 (k / 8), B alike, item k % 8
+//   result         D[i][j] lane j + 16 (i / 4), item i % 4
+// ---------------------------------------------------------------------------
+
+// tanh for activations that are rounded to bfloat16: 1 - 2 / (e^2x + 1), and below 1/4, where
+// that cancels, x + x^3 (c0 + c1 x^2) (least-squares fit of (tanh x - x) / x^3, reweighted to
+// equal ripple).  Relative error at most 5.3e-7 over all single-precision numbers, against
+// the rounding's 2e-3, without branches and in 17 vector operations' time; tanhf (1.5e-7)
+// takes about three times that.
+__device__ __forceinline__ float tanh_bf16(float x) {
+    const float z = x * x;
+    const float t = fmaf(-2.f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.8853900817779268f) + 1.f), 1.f);
+    const float p = fmaf(z, 0.12876420190194154f, -0.33324571367681377f);
+    return fabsf(x) < 0.25f ? fmaf(x * z, p, x) : t;
 }
 
-__global__ __launch_bounds__(kThr) void k_mlp_forward_mfma(const float* __restrict__ w, const float* __restrict__ X,
-                                                           int64_t rows, float* __restrict__ Y) {
-    __shared__ __align__(16) short sW2t[kH * kW2tPitch];   // sW2t[n * pitch + k] = bf16(W2[k][n])
-    __shared__ float sW1[kIn * kH];
-    __shared__ float sb1[kH], sb2[kH];
-    __shared__ float sW3[kH * kOut];
-    __shared__ float sb3[kOut];
-    const int t = threadIdx.x;
-    for (int i = t; i < kH * kH; i += kThr) sW2t[(i % kH) * kW2tPitch + i / kH] = bf16_bits(w[off_W2 + i]);
-    for (int i = t; i < kIn * kH; i += kThr) sW1[i] = bf16_round(w[i]);
-    for (int i = t; i < kH * kOut; i += kThr) sW3[i] = bf16_round(w[off_W3 + i]);
+// W3[c..c+3][0..2] (12 floats, 16-byte aligned)
+__device__ __forceinline__ void load_w3(const float* sW3, int c, float* w3) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(sW3 + kOut * c + 4 * q);
+#pragma unroll
+        for (int s = 0; s < 4; s++) w3[4 * q + s] = v[s];
+    }
+}
+
+// sums over the four lane groups of a row, in every one of them
+__device__ __forceinline__ void sum_groups(float* y) {
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1)
+#pragma unroll
+        for (int j = 0; j < kOut; j++) y[j] += __shfl_xor(y[j], o, 64);
+}
+
+// ---------------------------------------------------------------------------
+// FP32 layers of one wave's 16 rows (FP32 matrix instructions: FP32 products and sums)
+// ---------------------------------------------------------------------------
+constexpr int kW2Pitch = kH + 4;   // floats per LDS row of W2: W2^T reads one value per lane, W2 four, no conflicts
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// this lane's W1 operands, kept for all tiles
+__device__ __forceinline__ void load_w1(const float* w, int i, int g, float (*w1)[2]) {
+#pragma unroll
+    for (int b = 0; b < kH / 16; b++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) w1[b][k] = w[(4 * k + g) * kH + 16 * b + i];
+}
+
+// a1 = tanh(W1^T x + b1); x0, x1: inputs g and 4 + g of the lane's row
+__device__ __forceinline__ void layer1(const float (*w1)[2], const float* sb1, int g, float x0, float x1, f32x4* a1) {
+#pragma unroll
+    for (int b = 0; b < kH / 16; b++) {
+        f32x4 acc = *reinterpret_cast<const f32x4*>(sb1 + 16 * b + 4 * g);
+        acc = mfma4(w1[b][0], x0, acc);
+        acc = mfma4(w1[b][1], x1, acc);
+#pragma unroll
+        for (int s = 0; s < 4; s++) a1[b][s] = tanhf(acc[s]);
+    }
+}
+
+// a2 = tanh(W2^T a1 + b2).  The lane's offset is hidden from the compiler, which would
+// otherwise keep W2 in registers across a workgroup's tiles and spill them.
+__device__ __forceinline__ void layer2(const float* sW2, const float* sb2, int i, int g, const f32x4* a1, f32x4* a2) {
+    int lane = 4 * g * kW2Pitch + i;
+    asm volatile("" : "+v"(lane));
+#pragma unroll
+    for (int n = 0; n < kH / 16; n++) a2[n] = *reinterpret_cast<const f32x4*>(sb2 + 16 * n + 4 * g);
+    // the next k-step's weights are requested before this one's products (the barrier keeps the
+    // compiler from moving the loads back to their use, where every pair of products waits)
+    float wk[2][kH / 16];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int n = 0; n < kH / 16; n++)
+            wk[k % 2][n] = sW2[lane + (16 * (k / 4) + k % 4) * kW2Pitch + 16 * n];
+    };
+    load(0);
+#pragma unroll
+    for (int k = 0; k < kH / 4; k++) {
+        if (k + 1 < kH / 4) load(k + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < kH / 16; n++) a2[n] = mfma4(wk[k % 2][n], a1[k / 4][k % 4], a2[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < kH / 16; n++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) a2[n][s] = tanhf(a2[n][s]);
+}
+
+// y = W3^T a2 of the lane's row (without the bias), in all four lane groups
+__device__ __forceinline__ void layer3(const float* sW3, int g, const f32x4* a2, float* y) {
+    y[0] = y[1] = y[2] = 0.f;
+#pragma unroll
+    for (int b = 0; b < kH / 16; b++) {
+        float w3[12];
+        load_w3(sW3, 16 * b + 4 * g, w3);
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int o = 0; o < kOut; o++) y[o] = fmaf(a2[b][s], w3[3 * s + o], y[o]);
+    }
+    sum_groups(y);
+}
+
+// ---------------------------------------------------------------------------
+// forward (FP32): W2 in LDS for all tiles of a workgroup, 16 rows per wave.
+// Bound by the FP32 matrix rate (2 x 128 x 128 flops per row) and the two tanh layers on the
+// vector ALUs, which four waves per SIMD overlap.  290,927 rows: 139 us,
+// 430 with 4 x 8 outputs per thread on the vector ALUs.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(4 * kThr) void k_mlp_forward(const float* __restrict__ w, const float* __restrict__ X,
+                                                          int64_t rows, float* __restrict__ Y) {
+    __shared__ __align__(16) float sW2[kH * kW2Pitch];
+    __shared__ __align__(16) float sb1[kH], sb2[kH], sW3[kH * kOut];
+    const int t = threadIdx.x, nt = blockDim.x;
+    for (int e = 4 * t; e < kH * kH; e += 4 * nt)
+        *reinterpret_cast<f32x4*>(sW2 + (e / kH) * kW2Pitch + e % kH) = *reinterpret_cast<const f32x4*>(w + off_W2 + e);
+    for (int e = t; e < kH * kOut; e += nt) sW3[e] = w[off_W3 + e];
     if (t < kH) {
         sb1[t] = w[off_b1 + t];
         sb2[t] = w[off_b2 + t];
     }
-    if (t < kOut) sb3[t] = w[off_b3 + t];
+    const int i = t % 16, g = (t % 64) / 16;
+    float w1[kH / 16][2];
+    load_w1(w, i, g, w1);
+    const float b3 = g < kOut ? w[off_b3 + g] : 0.f;
     __syncthreads();
-    const int wv = t / 64, lane = t % 64;
-    const int li = lane % 16, lk = lane / 16;
-    const int64_t ntiles = (rows + kTile - 1) / kTile;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t r0 = tile * kTile + wv * 16;
-        // ---- layer 1 into the A operands ----
-        const int64_t ra = r0 + li;
-        float x[kIn];
-#pragma unroll
-        for (int k = 0; k < kIn; k++) x[k] = (ra < rows) ? bf16_round(X[ra * kIn + k]) : 0.f;
-        bf16x4 a[kH / 16];
-#pragma unroll
-        for (int ks = 0; ks < kH / 16; ks++)
-#pragma unroll 1
-            for (int j = 0; j < 4; j++) {
-                const int c = 16 * ks + 4 * lk + j;
-                float s = sb1[c];
-#pragma unroll
-                for (int k = 0; k < kIn; k++) s += x[k] * sW1[k * kH + c];
-                a[ks][j] = bf16_bits(tanhf(s));
-            }
-        // ---- layers 2 (matrix cores) and 3, one 16-column block of layer 2 at a time ----
-        float y[4][kOut];
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-            for (int o = 0; o < kOut; o++) y[r][o] = 0.f;
-#pragma unroll 1
-        for (int nb = 0; nb < kH / 16; nb++) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < kH / 16; ks++) {
-                const bf16x4 b = *reinterpret_cast<const bf16x4*>(&sW2t[(16 * nb + li) * kW2tPitch + 16 * ks + 4 * lk]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[ks], b, acc, 0, 0, 0);
-            }
-            const int n = 16 * nb + li;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const float h = bf16_round(tanhf(acc[r] + sb2[n]));
-#pragma unroll
-                for (int o = 0; o < kOut; o++) y[r][o] += h * sW3[n * kOut + o];
-            }
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1)
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int o = 0; o < kOut; o++) y[r][o] += __shfl_xor(y[r][o], off, 16);
-        if (li == 0)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int64_t row = r0 + 4 * lk + r;
-                if (row < rows)
-#pragma unroll
-                    for (int o = 0; o < kOut; o++) Y[row * kOut + o] = y[r][o] + sb3[o];
-            }
+    const int64_t ntiles = (rows + kWaveRows - 1) / kWaveRows, step = (int64_t)gridDim.x * (nt / 64);
+    for (int64_t tile = (int64_t)blockIdx.x * (nt / 64) + t / 64; tile < ntiles; tile += step) {
+        const int64_t r = tile * kWaveRows + i;
+        const bool in = r < rows;
+        f32x4 a1[kH / 16], a2[kH / 16];
+        float y[kOut];
+        layer1(w1, sb1, g, in ? X[r * kIn + g] : 0.f, in ? X[r * kIn + 4 + g] : 0.f, a1);
+        layer2(sW2, sb2, i, g, a1, a2);
+        layer3(sW3, g, a2, y);
+        if (in && g < kOut) Y[r * kOut + g] = (g == 0 ? y[0] : g == 1 ? y[1] : y[2]) + b3;
     }
 }
 
 // ---------------------------------------------------------------------------
-// backward, activation part: dY = 2 (Y - T) / (3 rows); dZ2 = (dY W3^T) (1 - A2^2);
-// dZ1 = (dZ2 W2^T) (1 - A1^2).  Per-block partial of the squared error.
+// bfloat16 inference: inputs, weights and both hidden activations rounded to bfloat16,
+// products and sums in FP32 on the matrix cores (layers 1 and 2) and the vector ALUs
+// (layer 3).  Layer 1 has k = 8, the instruction 16: the two upper lane groups hold zeros.
+// W2^T is stored in LDS with k permuted so that a lane's eight values of a 16x16x32 step,
+// columns 32 p + 4 g + s and 32 p + 16 + 4 g + s, are 16 contiguous bytes.
+// Bound by the 256 tanh per row (17 of the about 25 vector operations per activation).
+// 290,927 rows: 40 us, 89 with layer 1 on the vector ALUs, tanhf and one k = 16 step per
+// instruction.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThr) void k_mlp_backward_act(const float* __restrict__ w, int64_t rows,
-                                                           const float* __restrict__ Y, const float* __restrict__ T,
-                                                           const float* __restrict__ A1g,
-                                                           const float* __restrict__ A2g, float* __restrict__ dYg,
-                                                           float* __restrict__ dZ2g, float* __restrict__ dZ1g,
-                                                           double* __restrict__ loss_part) {
-    __shared__ float sW2[kH * kPad];   // padded: the W2^T product walks rows of W2
-    __shared__ float sW3[kH * kOut];
-    __shared__ float sdY[kTile * kOut];
-    __shared__ float sZ[kTile * kPad];
-    __shared__ double sl[kThr / 64];
-    const int t = threadIdx.x;
-    for (int i = t; i < kH * kH; i += kThr) sW2[(i / kH) * kPad + (i % kH)] = w[off_W2 + i];
-    for (int i = t; i < kH * kOut; i += kThr) sW3[i] = w[off_W3 + i];
-    __syncthreads();
-    const int rg = t / 16, cg = t % 16;
-    const int64_t ntiles = (rows + kTile - 1) / kTile;
-    const float scale = 2.0f / (float)(3 * rows);
-    double lsum = 0.0;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t r0 = tile * kTile;
-        if (t < kTile * kOut) {
-            const int64_t r = r0 + t / kOut;
-            float d = 0.f;
-            if (r < rows) {
-                const float e = Y[r * kOut + t % kOut] - T[r * kOut + t % kOut];
-                lsum += (double)e * (double)e;
-                d = scale * e;
-                dYg[r * kOut + t % kOut] = d;
-            }
-            sdY[t] = d;
-        }
-        __syncthreads();
-        // dZ2 for rows rg*4..+4, columns cg*8..+8
+constexpr int kW2tPitch = kH + 8;   // bf16 per row of the transposed W2 (spreads the lanes over banks)
+
+__global__ __launch_bounds__(4 * kThr) void k_mlp_forward_bf16(const float* __restrict__ w,
+                                                               const float* __restrict__ X, int64_t rows,
+                                                               float* __restrict__ Y) {
+    __shared__ __align__(16) __bf16 sW2t[kH * kW2tPitch];
+    __shared__ __align__(16) float sb1[kH], sb2[kH], sW3[kH * kOut];
+    const int t = threadIdx.x, nt = blockDim.x;
+    for (int e = t; e < kH * kH / 4; e += nt) {
+        const int n = e % kH, k = 4 * (e / kH);   // four values of column n
+        bf16x4 v;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int rr = rg * 4 + i;
-            const int64_t r = r0 + rr;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int c = cg * 8 + j;
-                float da = 0.f;
-#pragma unroll
-                for (int o = 0; o < kOut; o++) da += sdY[rr * kOut + o] * sW3[c * kOut + o];
-                const float a2 = (r < rows) ? A2g[r * kH + c] : 0.f;
-                const float dz = da * (1.f - a2 * a2);
-                sZ[rr * kPad + c] = dz;
-                if (r < rows) dZ2g[r * kH + c] = dz;
-            }
-        }
-        __syncthreads();
-        // dZ1 = (dZ2 W2^T)(1 - A1^2): dA1[r][c] = sum_k dZ2[r][k] W2[c][k]
-        float acc[4][8];
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) acc[i][j] = 0.f;
-        for (int k = 0; k < kH; k++) {
-            float a[4], b[8];
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = sZ[(rg * 4 + i) * kPad + k];
-#pragma unroll
-            for (int j = 0; j < 8; j++) b[j] = sW2[(cg * 8 + j) * kPad + k];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc[i][j] += a[i] * b[j];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int64_t r = r0 + rg * 4 + i;
-            if (r >= rows) continue;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int c = cg * 8 + j;
-                const float a1 = A1g[r * kH + c];
-                dZ1g[r * kH + c] = acc[i][j] * (1.f - a1 * a1);
-            }
-        }
-        __syncthreads();   // sZ / sdY are rewritten by the next tile
+        for (int s = 0; s < 4; s++) v[s] = (__bf16)w[off_W2 + (k + s) * kH + n];
+        const int kp = (k & ~31) + 8 * ((k % 16) / 4) + 4 * ((k / 16) % 2);
+        *reinterpret_cast<bf16x4*>(sW2t + n * kW2tPitch + kp) = v;
     }
-    // block partial of the squared error
+    for (int e = t; e < kH * kOut; e += nt) sW3[e] = (float)(__bf16)w[off_W3 + e];
+    if (t < kH) {
+        sb1[t] = w[off_b1 + t];
+        sb2[t] = w[off_b2 + t];
+    }
+    const int i = t % 16, g = (t % 64) / 16;
+    bf16x4 w1[kH / 16];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
-    if (t % 64 == 0) sl[t / 64] = lsum;
+    for (int b = 0; b < kH / 16; b++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) w1[b][s] = (__bf16)(g < 2 ? w[(4 * g + s) * kH + 16 * b + i] : 0.f);
+    const float b3 = g < kOut ? w[off_b3 + g] : 0.f;
     __syncthreads();
+    const int64_t ntiles = (rows + kWaveRows - 1) / kWaveRows, step = (int64_t)gridDim.x * (nt / 64);
+    for (int64_t tile = (int64_t)blockIdx.x * (nt / 64) + t / 64; tile < ntiles; tile += step) {
+        const int64_t r = tile * kWaveRows + i;
+        const bool in = r < rows;
+        bf16x4 x;
+#pragma unroll
+        for (int s = 0; s < 4; s++) x[s] = (__bf16)(in && g < 2 ? X[r * kIn + 4 * g + s] : 0.f);
+        bf16x8 a1[kH / 32];
+#pragma unroll
+        for (int p = 0; p < kH / 32; p++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int b = 2 * p + h;
+                f32x4 acc = *reinterpret_cast<const f32x4*>(sb1 + 16 * b + 4 * g);
+                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, w1[b]),
+                                                                __builtin_bit_cast(s16x4, x), acc, 0, 0, 0);
+#pragma unroll
+                for (int s = 0; s < 4; s++) a1[p][4 * h + s] = (__bf16)tanh_bf16(acc[s]);
+            }
+        float y[kOut] = {0.f, 0.f, 0.f};
+#pragma unroll 2
+        for (int n = 0; n < kH / 16; n++) {
+            f32x4 acc = *reinterpret_cast<const f32x4*>(sb2 + 16 * n + 4 * g);
+#pragma unroll
+            for (int p = 0; p < kH / 32; p++) {
+                const bf16x8 a = *reinterpret_cast<const bf16x8*>(sW2t + (16 * n + i) * kW2tPitch + 32 * p + 8 * g);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, a1[p], acc, 0, 0, 0);
+            }
+            float w3[12];
+            load_w3(sW3, 16 * n + 4 * g, w3);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const float h = (float)(__bf16)tanh_bf16(acc[s]);
+#pragma unroll
+                for (int o = 0; o < kOut; o++) y[o] = fmaf(h, w3[3 * s + o], y[o]);
+            }
+        }
+        sum_groups(y);
+        if (in && g < kOut) Y[r * kOut + g] = (g == 0 ? y[0] : g == 1 ? y[1] : y[2]) + b3;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// training pass: forward, dY = 2 (Y - T) / (3 rows), dZ2 = (dY W3^T) (1 - A2^2),
+// dZ1 = (dZ2 W2^T) (1 - A1^2), and the workgroup's partial of every gradient and of the
+// squared error, in one kernel.  A workgroup of four waves runs over 64-row tiles; a wave
+// keeps its 16 rows' activations and their gradients in registers and passes them through
+// LDS only as operands of the gradients' contractions over the rows:
+//   W2: A1^T dZ2, each wave 32 x 128 of it in accumulators for all tiles
+//   W1, b1: dZ1^T [X 1],  W3: A2^T dY,  b2: dZ2^T 1   with [X 1 dY] as one 16-column operand
+// Bound by the FP32 matrix rate (6 x 128 x 128 flops per row; one wave per SIMD, since the
+// LDS holds one workgroup) and the tanh between the products.  The activations that seven
+// kernels wrote and read (2 KB per row, up to three times) stay on the chip.
+// 31,000 rows: 67 us and 5 for the sum of the partials; the seven kernels took 606.
+// ---------------------------------------------------------------------------
+constexpr int kActPitch = kH + 16;   // floats per row of the activations in LDS: column reads without conflicts
+constexpr int64_t kPartPitch = (n_weights() + 63) / 64 * 64;
+
+__global__ __launch_bounds__(kThr) void k_mlp_train(const float* __restrict__ w, const float* __restrict__ X,
+                                                    const float* __restrict__ T, int64_t rows,
+                                                    float* __restrict__ part, double* __restrict__ loss_part) {
+    __shared__ __align__(16) float sW2[kH * kW2Pitch];
+    __shared__ __align__(16) float sA[kTile * kActPitch], sZ[kTile * kActPitch];
+    __shared__ __align__(16) float sB[kTile * 16];   // columns 0..7 X, 8 one, 9..11 dY
+    __shared__ __align__(16) float sb1[kH], sb2[kH], sW3[kH * kOut];
+    __shared__ double sl[kThr / 64];
+    __shared__ float sg[kThr / 64][kOut];
+    const int t = threadIdx.x;
+    for (int e = 4 * t; e < kH * kH; e += 4 * kThr)
+        *reinterpret_cast<f32x4*>(sW2 + (e / kH) * kW2Pitch + e % kH) = *reinterpret_cast<const f32x4*>(w + off_W2 + e);
+    for (int e = t; e < kH * kOut; e += kThr) sW3[e] = w[off_W3 + e];
+    if (t < kH) {
+        sb1[t] = w[off_b1 + t];
+        sb2[t] = w[off_b2 + t];
+    }
+    const int wv = t / 64, i = t % 16, g = (t % 64) / 16;
+    float w1[kH / 16][2], b3[kOut];
+    load_w1(w, i, g, w1);
+#pragma unroll
+    for (int o = 0; o < kOut; o++) b3[o] = w[off_b3 + o];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 gW2[2][kH / 16], gb2[2], gW3[2], gW1[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        gb2[h] = gW3[h] = gW1[h] = zero;
+#pragma unroll
+        for (int n = 0; n < kH / 16; n++) gW2[h][n] = zero;
+    }
+    float gb3[kOut] = {0.f, 0.f, 0.f};
+    double lsum = 0.0;
+    const float scale = 2.0f / (float)(3 * rows);
+    __syncthreads();
+    const int64_t ntiles = (rows + kTile - 1) / kTile;
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int lr = kWaveRows * wv + i;   // the lane's row in the tile
+        const int64_t r = tile * kTile + lr;
+        const bool in = r < rows;
+        const float x0 = in ? X[r * kIn + g] : 0.f, x1 = in ? X[r * kIn + 4 + g] : 0.f;
+        f32x4 a1[kH / 16], a2[kH / 16], z2[kH / 16], z1[kH / 16];
+        float y[kOut], d[kOut];
+        layer1(w1, sb1, g, x0, x1, a1);
+        layer2(sW2, sb2, i, g, a1, a2);
+        layer3(sW3, g, a2, y);
+#pragma unroll
+        for (int o = 0; o < kOut; o++) {
+            const float e = in ? (y[o] + b3[o]) - T[r * kOut + o] : 0.f;
+            d[o] = scale * e;
+            if (g == 0) {
+                lsum += (double)e * (double)e;
+                gb3[o] += d[o];
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kH / 16; b++) {
+            float w3[12];
+            load_w3(sW3, 16 * b + 4 * g, w3);
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const float da = d[0] * w3[3 * s] + d[1] * w3[3 * s + 1] + d[2] * w3[3 * s + 2];
+                z2[b][s] = da * (1.f - a2[b][s] * a2[b][s]);
+            }
+        }
+        // dA1^T[c][row] = sum_k W2[c][k] dZ2^T[k][row]
+#pragma unroll
+        for (int n = 0; n < kH / 16; n++) z1[n] = zero;
+        {
+            f32x4 wk[2][kH / 16];
+            int lane = i * kW2Pitch + 4 * g;
+            asm volatile("" : "+v"(lane));   // as in layer2
+            auto load = [&](int b) {
+#pragma unroll
+                for (int n = 0; n < kH / 16; n++)
+                    wk[b % 2][n] = *reinterpret_cast<const f32x4*>(sW2 + lane + 16 * n * kW2Pitch + 16 * b);
+            };
+            load(0);
+#pragma unroll
+            for (int b = 0; b < kH / 16; b++) {
+                if (b + 1 < kH / 16) load(b + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+#pragma unroll
+                    for (int n = 0; n < kH / 16; n++) z1[n] = mfma4(wk[b % 2][n][s], z2[b][s], z1[n]);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kH / 16; b++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) z1[b][s] *= 1.f - a1[b][s] * a1[b][s];
+        __syncthreads();   // the last tile's operands are consumed
+        sB[16 * lr + g] = x0;
+        sB[16 * lr + 4 + g] = x1;
+        sB[16 * lr + 8 + g] = g == 0 ? 1.f : g == 1 ? d[0] : g == 2 ? d[1] : d[2];
+        sB[16 * lr + 12 + g] = 0.f;
+#pragma unroll
+        for (int b = 0; b < kH / 16; b++) {
+            *reinterpret_cast<f32x4*>(sA + lr * kActPitch + 16 * b + 4 * g) = a1[b];
+            *reinterpret_cast<f32x4*>(sZ + lr * kActPitch + 16 * b + 4 * g) = z2[b];
+        }
+        __syncthreads();
+        {
+            float va[2][2], vz[2][kH / 16], vb[2][2], v1[2];
+            auto load = [&](int j) {
+                const float* ra = sA + (4 * j + g) * kActPitch + i;
+                const float* rz = sZ + (4 * j + g) * kActPitch + i;
+                const int u = j % 2;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    va[u][h] = ra[32 * wv + 16 * h];
+                    vb[u][h] = rz[32 * wv + 16 * h];
+                }
+#pragma unroll
+                for (int n = 0; n < kH / 16; n++) vz[u][n] = rz[16 * n];
+                v1[u] = sB[16 * (4 * j + g) + i];
+            };
+            load(0);
+#pragma unroll
+            for (int j = 0; j < kTile / 4; j++) {
+                const int u = j % 2;
+                if (j + 1 < kTile / 4) load(j + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+#pragma unroll
+                    for (int n = 0; n < kH / 16; n++) gW2[h][n] = mfma4(va[u][h], vz[u][n], gW2[h][n]);
+                    gb2[h] = mfma4(vb[u][h], v1[u], gb2[h]);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < kH / 16; b++) {
+            *reinterpret_cast<f32x4*>(sA + lr * kActPitch + 16 * b + 4 * g) = a2[b];
+            *reinterpret_cast<f32x4*>(sZ + lr * kActPitch + 16 * b + 4 * g) = z1[b];
+        }
+        __syncthreads();
+        {
+            constexpr int kAhead = 4;   // k-steps loaded together: each has only four products
+            float v[2][kAhead], x[2][kAhead][2], z[2][kAhead][2];
+            auto load = [&](int j) {
+#pragma unroll
+                for (int q = 0; q < kAhead; q++) {
+                    const int row = 4 * (kAhead * j + q) + g;
+                    v[j % 2][q] = sB[16 * row + i];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        x[j % 2][q][h] = sA[row * kActPitch + 32 * wv + 16 * h + i];
+                        z[j % 2][q][h] = sZ[row * kActPitch + 32 * wv + 16 * h + i];
+                    }
+                }
+            };
+            load(0);
+#pragma unroll
+            for (int j = 0; j < kTile / 4 / kAhead; j++) {
+                if (j + 1 < kTile / 4 / kAhead) load(j + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int q = 0; q < kAhead; q++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        gW3[h] = mfma4(x[j % 2][q][h], v[j % 2][q], gW3[h]);
+                        gW1[h] = mfma4(z[j % 2][q][h], v[j % 2][q], gW1[h]);
+                    }
+            }
+        }
+    }
+    // partials, laid out like the weights
+    float* out = part + (int64_t)blockIdx.x * kPartPitch;
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int c = 32 * wv + 16 * h + 4 * g + s;
+#pragma unroll
+            for (int n = 0; n < kH / 16; n++) out[off_W2 + c * kH + 16 * n + i] = gW2[h][n][s];
+            if (i < kIn) out[i * kH + c] = gW1[h][s];
+            if (i == kIn) {
+                out[off_b1 + c] = gW1[h][s];
+                out[off_b2 + c] = gb2[h][s];
+            }
+            if (i > kIn && i <= kIn + kOut) out[off_W3 + c * kOut + i - kIn - 1] = gW3[h][s];
+        }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lsum += __shfl_xor(lsum, o, 64);
+#pragma unroll
+        for (int j = 0; j < kOut; j++) gb3[j] += __shfl_xor(gb3[j], o, 64);
+    }
+    if (t % 64 == 0) {
+        sl[wv] = lsum;
+#pragma unroll
+        for (int j = 0; j < kOut; j++) sg[wv][j] = gb3[j];
+    }
+    __syncthreads();
+    if (t < kOut) out[off_b3 + t] = sg[0][t] + sg[1][t] + sg[2][t] + sg[3][t];
     if (t == 0) loss_part[blockIdx.x] = sl[0] + sl[1] + sl[2] + sl[3];
 }
 
-// ---------------------------------------------------------------------------
-// weight gradient G[Ka][Kb] = A^T B and bias gradient gb[Kb] = sum_r B[r][:]
-// over rows, in kGradBlocks contiguous row ranges (partials, fixed order).
-// Thread t owns the entries t, t + 256, ... of G (and of gb).
-// ---------------------------------------------------------------------------
-template <int KA, int KB>
-__global__ __launch_bounds__(kThr) void k_mlp_wgrad(const float* __restrict__ A, const float* __restrict__ B,
-                                                    int64_t rows, float* __restrict__ part) {
-    constexpr int NG = KA * KB;
-    constexpr int PER = (NG + kThr - 1) / kThr;
-    constexpr int CH = 16;   // rows staged per pass
-    __shared__ float sa[CH * KA];
-    __shared__ float sb[CH * KB];
-    const int t = threadIdx.x;
-    const int64_t per_block = (rows + gridDim.x - 1) / gridDim.x;
-    const int64_t lo = (int64_t)blockIdx.x * per_block;
-    const int64_t hi = std::min<int64_t>(rows, lo + per_block);
-    float g[PER];
-#pragma unroll
-    for (int q = 0; q < PER; q++) g[q] = 0.f;
-    float gb = 0.f;
-    for (int64_t r0 = lo; r0 < hi; r0 += CH) {
-        const int nr = (int)std::min<int64_t>(CH, hi - r0);
-        for (int i = t; i < CH * KA; i += kThr) sa[i] = (i / KA < nr) ? A[(r0 + i / KA) * KA + i % KA] : 0.f;
-        for (int i = t; i < CH * KB; i += kThr) sb[i] = (i / KB < nr) ? B[(r0 + i / KB) * KB + i % KB] : 0.f;
-        __syncthreads();
-        for (int rr = 0; rr < CH; rr++) {
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int e = t + q * kThr;
-                if (e < NG) g[q] += sa[rr * KA + e / KB] * sb[rr * KB + e % KB];
-            }
-            if (t < KB) gb += sb[rr * KB + t];
-        }
-        __syncthreads();
-    }
-    float* out = part + (int64_t)blockIdx.x * (NG + KB);
-#pragma unroll
-    for (int q = 0; q < PER; q++) {
-        const int e = t + q * kThr;
-        if (e < NG) out[e] = g[q];
-    }
-    if (t < KB) out[NG + t] = gb;
-}
-
-// sum of the kGradBlocks partials into grad[off_w..] and grad[off_b..]
-__global__ __launch_bounds__(kThr) void k_mlp_wgrad_reduce(const float* __restrict__ part, int nblk, int ng, int kb,
-                                                           float* __restrict__ gw, float* __restrict__ gbias) {
-    const int e = blockIdx.x * kThr + threadIdx.x;
-    if (e >= ng + kb) return;
+// sum of the workgroups' partial gradients: 32 weights per workgroup, eight threads each over
+// every eighth partial, then the eight in order
+__global__ __launch_bounds__(kThr) void k_mlp_grad_reduce(const float* __restrict__ part, int nblk,
+                                                          float* __restrict__ grad) {
+    __shared__ float sh[kThr / 32][32];
+    const int t = threadIdx.x % 32, seg = threadIdx.x / 32;
+    const int e = blockIdx.x * 32 + t;   // < kPartPitch
     float s = 0.f;
-    for (int b = 0; b < nblk; b++) s += part[(int64_t)b * (ng + kb) + e];
-    if (e < ng)
-        gw[e] = s;
-    else
-        gbias[e - ng] = s;
+#pragma unroll 8
+    for (int b = seg; b < nblk; b += kThr / 32) s += part[(int64_t)b * kPartPitch + e];
+    sh[seg][t] = s;
+    __syncthreads();
+    if (seg == 0 && e < n_weights()) {
+#pragma unroll
+        for (int q = 1; q < kThr / 32; q++) s += sh[q][t];
+        grad[e] = s;
+    }
 }
 
 __global__ __launch_bounds__(kThr) void k_adam(int64_t P, float* __restrict__ w, const float* __restrict__ g,
@@ -457,8 +577,6 @@ struct cmg_mlp {
     cmg_ctx* c = nullptr;
     int device = 0;
     DevBuf w, g, m, v, part, loss_part, tact_node;
-    DevBuf A1, A2, dY, dZ1, dZ2, Yt;
-    int64_t cap_rows = 0;
     int adam_t = 0;
     double s_inc = 1.0, s_p = 1.0, s_t = 1.0;
     double* h_pin = nullptr;
@@ -469,22 +587,15 @@ struct cmg_mlp {
 
 namespace {
 
-int ensure_rows(cmg_mlp* m, int64_t rows) {
-    if (rows <= m->cap_rows) return CMG_SUCCESS;
-    const int64_t cap = std::max<int64_t>(rows, 2 * m->cap_rows);
-    CMG_TRY(alloc(m->A1, (size_t)cap * kH * sizeof(float)));
-    CMG_TRY(alloc(m->A2, (size_t)cap * kH * sizeof(float)));
-    CMG_TRY(alloc(m->dZ1, (size_t)cap * kH * sizeof(float)));
-    CMG_TRY(alloc(m->dZ2, (size_t)cap * kH * sizeof(float)));
-    CMG_TRY(alloc(m->dY, (size_t)cap * kOut * sizeof(float)));
-    CMG_TRY(alloc(m->Yt, (size_t)cap * kOut * sizeof(float)));
-    m->cap_rows = cap;
-    return CMG_SUCCESS;
-}
-
-unsigned fwd_blocks(int64_t rows) {
-    const int64_t tiles = (rows + kTile - 1) / kTile;
-    return (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, 1024));
+// one 16-row tile per wave up to a wave on every SIMD, then sixteen per workgroup, so that
+// a workgroup's copy of the weights serves more rows, in at most one workgroup per CU
+struct ForwardShape {
+    unsigned blocks, threads;
+};
+ForwardShape forward_shape(int64_t rows) {
+    const int64_t tiles = (rows + kWaveRows - 1) / kWaveRows;
+    const int per = tiles > 4 * 256 ? 16 : 4;
+    return {(unsigned)std::min<int64_t>((tiles + per - 1) / per, 256), (unsigned)(64 * per)};
 }
 
 }  // namespace
@@ -502,10 +613,10 @@ int cmg_mlp_create(cmg_ctx* c, int32_t hidden, uint64_t seed, cmg_mlp** out) {
     m->device = c->device;
     const int64_t P = n_weights();
     for (DevBuf* b : {&m->w, &m->g, &m->m, &m->v}) CMG_TRY(alloc(*b, P * sizeof(float)));
-    CMG_TRY(alloc(m->part, (size_t)kGradBlocks * (kH * kH + kH) * sizeof(float)));
-    CMG_TRY(alloc(m->loss_part, 1024 * sizeof(double)));
+    CMG_TRY(alloc(m->part, (size_t)kTrainBlocks * kPartPitch * sizeof(float)));
+    CMG_TRY(alloc(m->loss_part, kTrainBlocks * sizeof(double)));
     CMG_TRY(alloc(m->tact_node, c->N * sizeof(double)));
-    CMG_HIP_CHECK(hipHostMalloc((void**)&m->h_pin, 1024 * sizeof(double), hipHostMallocDefault));
+    CMG_HIP_CHECK(hipHostMalloc((void**)&m->h_pin, kTrainBlocks * sizeof(double), hipHostMallocDefault));
     // Glorot-uniform weights, zero biases (seeded host generator)
     std::vector<float> w(P, 0.f);
     std::mt19937_64 gen(seed);
@@ -591,11 +702,11 @@ int cmg_mlp_forward(cmg_mlp* m, const float* X, int64_t rows, int32_t bf16, floa
     if (rows <= 0) return CMG_SUCCESS;
     CMG_HIP_CHECK(hipSetDevice(m->c->device));
     hipStream_t s = m->c->stream;
+    const ForwardShape sh = forward_shape(rows);
     if (bf16)
-        hipLaunchKernelGGL(k_mlp_forward_mfma, dim3(fwd_blocks(rows)), dim3(kThr), 0, s, m->w.as<float>(), X, rows, Y);
+        hipLaunchKernelGGL(k_mlp_forward_bf16, dim3(sh.blocks), dim3(sh.threads), 0, s, m->w.as<float>(), X, rows, Y);
     else
-        hipLaunchKernelGGL(k_mlp_forward, dim3(fwd_blocks(rows)), dim3(kThr), 0, s, m->w.as<float>(), X, rows, Y,
-                           nullptr, nullptr);
+        hipLaunchKernelGGL(k_mlp_forward, dim3(sh.blocks), dim3(sh.threads), 0, s, m->w.as<float>(), X, rows, Y);
     CMG_HIP_CHECK(hipGetLastError());
     return CMG_SUCCESS;
 }
@@ -605,31 +716,13 @@ int cmg_mlp_loss_grad(cmg_mlp* m, const float* X, const float* T, int64_t rows, 
     if (rows <= 0) return fail("cmg_mlp_loss_grad: no rows");
     cmg_ctx* c = m->c;
     CMG_HIP_CHECK(hipSetDevice(c->device));
-    CMG_TRY(ensure_rows(m, rows));
     hipStream_t s = c->stream;
-    const float* w = m->w.as<float>();
     float* g = m->g.as<float>();
-    const unsigned nb = fwd_blocks(rows);
-    hipLaunchKernelGGL(k_mlp_forward, dim3(nb), dim3(kThr), 0, s, w, X, rows, m->Yt.as<float>(),
-                       m->A1.as<float>(), m->A2.as<float>());
-    hipLaunchKernelGGL(k_mlp_backward_act, dim3(nb), dim3(kThr), 0, s, w, rows, m->Yt.as<float>(), T,
-                       m->A1.as<float>(), m->A2.as<float>(), m->dY.as<float>(), m->dZ2.as<float>(),
-                       m->dZ1.as<float>(), m->loss_part.as<double>());
-    float* part = m->part.as<float>();
-    // dW3 = A2^T dY, db3
-    hipLaunchKernelGGL((k_mlp_wgrad<kH, kOut>), dim3(kGradBlocks), dim3(kThr), 0, s, m->A2.as<float>(),
-                       m->dY.as<float>(), rows, part);
-    hipLaunchKernelGGL(k_mlp_wgrad_reduce, dim3(grid_for(kH * kOut + kOut)), dim3(kThr), 0, s, part, kGradBlocks,
-                       kH * kOut, kOut, g + off_W3, g + off_b3);
-    // dW2 = A1^T dZ2, db2
-    hipLaunchKernelGGL((k_mlp_wgrad<kH, kH>), dim3(kGradBlocks), dim3(kThr), 0, s, m->A1.as<float>(),
-                       m->dZ2.as<float>(), rows, part);
-    hipLaunchKernelGGL(k_mlp_wgrad_reduce, dim3(grid_for(kH * kH + kH)), dim3(kThr), 0, s, part, kGradBlocks, kH * kH,
-                       kH, g + off_W2, g + off_b2);
-    // dW1 = X^T dZ1, db1
-    hipLaunchKernelGGL((k_mlp_wgrad<kIn, kH>), dim3(kGradBlocks), dim3(kThr), 0, s, X, m->dZ1.as<float>(), rows, part);
-    hipLaunchKernelGGL(k_mlp_wgrad_reduce, dim3(grid_for(kIn * kH + kH)), dim3(kThr), 0, s, part, kGradBlocks,
-                       kIn * kH, kH, g, g + off_b1);
+    const unsigned nb = (unsigned)std::min<int64_t>((rows + kTile - 1) / kTile, kTrainBlocks);
+    hipLaunchKernelGGL(k_mlp_train, dim3(nb), dim3(kThr), 0, s, m->w.as<float>(), X, T, rows, m->part.as<float>(),
+                       m->loss_part.as<double>());
+    hipLaunchKernelGGL(k_mlp_grad_reduce, dim3((unsigned)(kPartPitch / 32)), dim3(kThr), 0, s, m->part.as<float>(),
+                       (int)nb, g);
     CMG_HIP_CHECK(hipGetLastError());
     CMG_HIP_CHECK(hipMemcpyAsync(m->h_pin, m->loss_part.p, nb * sizeof(double), hipMemcpyDeviceToHost, s));
     if (grad_host) CMG_HIP_CHECK(hipMemcpyAsync(grad_host, g, n_weights() * sizeof(float), hipMemcpyDeviceToHost, s));
