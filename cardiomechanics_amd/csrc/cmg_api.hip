@@ -303,7 +303,7 @@ int cmg_create(const cmg_mesh* mesh, const cmg_material* materials, int32_t n_ma
     CMG_TRY(upload(c->bcmask, c->h_bc.data(), N, s));
     CMG_TRY(upload(c->Xref, mesh->ref_coords, 3 * N, s));
     CMG_TRY(alloc(c->w, E * sizeof(double)));
-    CMG_TRY(alloc(c->dNdX, (size_t)c->nqp * npe * 3 * E * sizeof(double)));
+    CMG_TRY(alloc(c->dNdX, (size_t)(npe == 10 ? 4 * kT10Grad : 12) * E * sizeof(double)));
     std::vector<double> wh(E);
     if (npe == 10) {
         DevBuf conn_aos;

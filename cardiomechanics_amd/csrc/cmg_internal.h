@@ -40,12 +40,14 @@ struct DevMaterial {
 // (one per spatial component pair i, j) per element, 7 elements per wave.
 constexpr int kTanElemsPerWave = 7;
 constexpr int kResidualBlock = 128;
+constexpr int kT10Grad = 13;   // values per T10 quadrature point from which dN/dX follows
 
 // Per-element data, structure-of-arrays: entry k of element e at [k * E + e].
 struct ElemArgs {
     int64_t E = 0;
     const int32_t* conn = nullptr;     // [npe][E]
-    const double* dNdX = nullptr;      // [nqp*npe*3][E]  reference dN/dX at the quadrature points
+    const double* dNdX = nullptr;      // reference gradients at the quadrature points: T10 [4*kT10Grad][E]
+                                       // (load_g), T4 [12][E] dN/dX
     const double* bases = nullptr;     // [nqp*9][E]      fibre frame (columns f, s, n) per quadrature point
     const double* w = nullptr;         // [E]  detJ/24 (T10) or volume (T4)
     const int32_t* matidx = nullptr;   // [E] or nullptr
@@ -97,7 +99,7 @@ void launch_element_residual(int npe, const ElemArgs& a, hipStream_t s);
 // with two 7-element groups per workgroup, so the quadrature stage fills 56 lanes of the first wave
 void launch_element_residual_tangent(int npe, bool fp32, const ElemArgs& a, hipStream_t s, int variant);
 void launch_surface(const SurfArgs& a, bool tangent, hipStream_t s);
-void launch_t10_shape(int64_t E, const int32_t* conn_aos, const double* X, double* dNdX_soa, double* w, hipStream_t s);
+void launch_t10_shape(int64_t E, const int32_t* conn_aos, const double* X, double* grad_soa, double* w, hipStream_t s);
 // Land17 commit: each Land17 element advances its state [8][E] in place from the
 // evaluation at its last quadrature point at coordinates a.x and time a.time
 void launch_land17_commit(int npe, const ElemArgs& a, double* state, hipStream_t s);

@@ -419,13 +419,61 @@ __device__ __forceinline__ void lane_M(const DevMaterial& m, const Law& L, const
     for (int r = 0; r < 9; r++) M[r] = (TT)Mm[r];
 }
 
+// dN/dX of T10 node k from the gradients' numerators v of the four barycentric coordinates
+// and fac = 4 / det J at the point (l1..l4), CBElementSolidT10.cpp:221-262
+__device__ __forceinline__ void t10_gradient(int k, const double* l, const double (*v)[3], double fac, double* g) {
+#pragma clang fp contract(off)
+    constexpr int A[6] = {0, 1, 2, 0, 1, 2}, B[6] = {1, 2, 0, 3, 3, 3};   // ends of the edge of node 4 + i
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        g[d] = k < 4 ? fac * (l[k & 3] - 0.25) * v[k & 3][d]
+                     : fac * (l[A[k < 4 ? 0 : k - 4]] * v[B[k < 4 ? 0 : k - 4]][d] +
+                              l[B[k < 4 ? 0 : k - 4]] * v[A[k < 4 ? 0 : k - 4]][d]);
+}
+
+// barycentric coordinates of the quadrature points: (qa, qb, qb, qb) and its permutations
+__device__ __forceinline__ double t10_qa() { return (5 + 3 * sqrt(5.0)) / 20; }
+__device__ __forceinline__ double t10_qb() { return (5 - sqrt(5.0)) / 20; }
+
+// T10: 13 stored values per point (v and fac) instead of the 30 gradients they give, bit for
+// bit the same numbers for 104 instead of 240 bytes per point
+__device__ __forceinline__ double load_t10(const ElemArgs& a, int64_t e, int q, double* l, double (*v)[3]) {
+    const int64_t E = a.E;
+    const double* p = a.dNdX + (int64_t)(kT10Grad * q) * E + e;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        l[i] = i == q ? t10_qa() : t10_qb();
+#pragma unroll
+        for (int d = 0; d < 3; d++) v[i][d] = p[(int64_t)(3 * i + d) * E];
+    }
+    return p[(int64_t)12 * E];
+}
+
 template <int NPE>
 __device__ __forceinline__ void load_g(const ElemArgs& a, int64_t e, int q, double (*g)[3]) {
     const int64_t E = a.E;
+    if constexpr (NPE == 10) {
+        double v[4][3], l[4];
+        const double fac = load_t10(a, e, q, l, v);
 #pragma unroll
-    for (int k = 0; k < NPE; k++)
+        for (int k = 0; k < 10; k++) t10_gradient(k, l, v, fac, g[k]);
+    } else {
 #pragma unroll
-        for (int d = 0; d < 3; d++) g[k][d] = a.dNdX[((int64_t)(q * NPE + k) * 3 + d) * E + e];
+        for (int k = 0; k < NPE; k++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) g[k][d] = a.dNdX[((int64_t)(q * NPE + k) * 3 + d) * E + e];
+    }
+}
+
+// the deformation gradient in the fibre frame B
+__device__ __forceinline__ void to_fibre_frame(const double* F, const double* B, double* Binv, double* Floc) {
+#pragma clang fp contract(off)
+    double Bt[9], BinvT[9], T1[9];
+    inv3(B, Binv);
+    tr3(B, Bt);
+    tr3(Binv, BinvT);
+    mul3(Bt, F, T1);
+    mul3(T1, BinvT, Floc);
 }
 
 template <int NPE>
@@ -442,12 +490,31 @@ __device__ __forceinline__ void local_F(const double* x, const double (*g)[3], c
             for (int k = 0; k < NPE; k++) s += g[k][j] * x[3 * k + i];
             F[3 * i + j] = s;
         }
-    double Bt[9], BinvT[9], T1[9];
-    inv3(B, Binv);
-    tr3(B, Bt);
-    tr3(Binv, BinvT);
-    mul3(Bt, F, T1);
-    mul3(T1, BinvT, Floc);
+    to_fibre_frame(F, B, Binv, Floc);
+}
+
+// The deformation gradient at a T10 point, node by node in local_F's order: a node's gradient
+// lives for its nine products only (60 registers fewer than all ten gradients at once)
+__device__ __forceinline__ void t10_F(const ElemArgs& a, int64_t e, const double* l, const double (*v)[3], double fac,
+                                      double* F) {
+#pragma clang fp contract(off)
+    double x[10][3];
+#pragma unroll
+    for (int k = 0; k < 10; k++) {
+        const int64_t n = a.conn[(int64_t)k * a.E + e];
+#pragma unroll
+        for (int c = 0; c < 3; c++) x[k][c] = a.x[3 * n + c];
+    }
+#pragma unroll
+    for (int r = 0; r < 9; r++) F[r] = 0.0;
+#pragma unroll
+    for (int k = 0; k < 10; k++) {
+        double g[3];
+        t10_gradient(k, l, v, fac, g);
+#pragma unroll
+        for (int r = 0; r < 9; r++) F[r] += g[r % 3] * x[k][r / 3];
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -577,6 +644,72 @@ __global__ __launch_bounds__(kResidualBlock) void k_residual(const ElemArgs a0) 
     for (int k = 0; k < NPE; k++)
 #pragma unroll
         for (int c = 0; c < 3; c++) fe[3 * k + c] = V * t[k][c];
+}
+
+// The T10 residual with the four quadrature points of an element in the four waves of a
+// workgroup (64 elements): four times the lanes and a quarter of the serial work per lane.
+// Every point's terms go through LDS and are summed in point order, so the forces equal
+// those of one lane per element bit for bit.  Bound by the FP64 operations of the point (about
+// 2,000, contraction off) and their latency: 154 registers and half of the terms in LDS
+// at a time let three workgroups share a CU.  Against one lane per element (256 registers and
+// spills, one wave per SIMD): 200k elements 69 / 109 us, 20k 14.2 / 22 us, 5k 9.4 / 19.5 us.
+constexpr int kSplitPitch = 65;   // elements per LDS row, padded
+
+template <bool LAND17>
+__global__ __launch_bounds__(256) void k_residual_t10(const ElemArgs a0) {
+#pragma clang fp contract(off)
+    __shared__ double sT[4][15][kSplitPitch];   // half of the 30 components at a time
+    ElemArgs a;
+    if (!batch_select(a0, a)) return;
+    const int q = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l = (int)(threadIdx.x & 63);
+    const int64_t e0 = (int64_t)blockIdx.x * 64, e = e0 + l;
+    const int64_t E = a.E;
+    double l4[4], v[4][3], fac = 0.0, P[9];
+    if (e < E) {
+        const DevMaterial& m = a.mats[a.matidx ? a.matidx[e] : 0];
+        double ts;
+        const double Ta = tension_of(m, a.time, a.tact[e], ts);
+        L17 l17s;
+        const L17* l17 = nullptr;
+        if (LAND17 && m.tension_fn == CMG_FN_LAND17) {
+            load_l17(a, e, a.matidx ? a.matidx[e] : 0, m, l17s);
+            l17 = &l17s;
+        }
+        double F[9], B[9], Binv[9], Floc[9];
+        fac = load_t10(a, e, q, l4, v);
+#pragma unroll
+        for (int r = 0; r < 9; r++) B[r] = a.bases[(int64_t)(q * 9 + r) * E + e];
+        t10_F(a, e, l4, v, fac, F);
+        to_fibre_frame(F, B, Binv, Floc);
+        Law L;
+        if (!eval_law(m, Floc, Ta, ts, false, L, l17)) atomicMin(a.corrupt, (int)e);
+        double FS[9], P1[9], BinvT[9], Bt[9], St[9];
+        mul3(Floc, L.S, FS);
+        tr3(FS, St);
+        tr3(Binv, BinvT);
+        tr3(B, Bt);
+        mul3(BinvT, St, P1);
+        mul3(P1, Bt, P);
+    }
+    const int n = (int)(E - e0 < 64 ? E - e0 : 64) * 15;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (h) __syncthreads();
+        if (e < E)
+#pragma unroll
+            for (int k = 0; k < 5; k++) {
+                double g[3];
+                t10_gradient(5 * h + k, l4, v, fac, g);
+#pragma unroll
+                for (int c = 0; c < 3; c++) sT[q][3 * k + c][l] = g[0] * P[0 + c] + g[1] * P[3 + c] + g[2] * P[6 + c];
+            }
+        __syncthreads();
+        for (int t = (int)threadIdx.x; t < n; t += 256) {
+            const int el = t / 15, r = t - 15 * el;
+            a.fe[(e0 + el) * 30 + 15 * h + r] =
+                a.w[e0 + el] * (((sT[0][r][el] + sT[1][r][el]) + sT[2][r][el]) + sT[3][r][el]);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1131,9 +1264,10 @@ __global__ __launch_bounds__(64) void k_surface(const SurfArgs a0, bool tangent)
     }
 }
 
-// dN/dX at the 4 quadrature points (SoA) and detJ/24 per element,
+// numerators of the barycentric gradients, 4 / det J and det J at a point of a T10 element,
 // CBElementSolidT10::CalcShapeFunctionDerivatives (:94-264)
-__device__ double t10_shape_point(const double* X, double l1, double l2, double l3, double l4, double* out) {
+__device__ double t10_shape_vectors(const double* X, double l1, double l2, double l3, double l4, double (*v)[3],
+                                    double& fac) {
 #pragma clang fp contract(off)
     double Jx[4], Jy[4], Jz[4];
     const double* c[10];
@@ -1162,42 +1296,30 @@ __device__ double t10_shape_point(const double* X, double l1, double l2, double 
                           D_(Jx, 2, 4) * D_(Jy, 1, 4) - D_(Jx, 1, 4) * D_(Jy, 2, 4),
                           D_(Jx, 1, 3) * D_(Jy, 2, 1) - D_(Jx, 1, 2) * D_(Jy, 3, 1)};
 #undef D_
-    const double fac = 4.0 / detJ;
+    fac = 4.0 / detJ;
     const double* comp[3] = {av, bv, cv};
-    for (int d = 0; d < 3; d++) {
-        const double* v = comp[d];
-        out[0 + d] = fac * (l1 - 0.25) * v[0];
-        out[3 + d] = fac * (l2 - 0.25) * v[1];
-        out[6 + d] = fac * (l3 - 0.25) * v[2];
-        out[9 + d] = fac * (l4 - 0.25) * v[3];
-        out[12 + d] = fac * (l1 * v[1] + l2 * v[0]);
-        out[15 + d] = fac * (l2 * v[2] + l3 * v[1]);
-        out[18 + d] = fac * (l3 * v[0] + l1 * v[2]);
-        out[21 + d] = fac * (l1 * v[3] + l4 * v[0]);
-        out[24 + d] = fac * (l2 * v[3] + l4 * v[1]);
-        out[27 + d] = fac * (l3 * v[3] + l4 * v[2]);
-    }
+    for (int d = 0; d < 3; d++)
+        for (int i = 0; i < 4; i++) v[i][d] = comp[d][i];
     return detJ;
 }
 
-__global__ void k_t10_shape(int64_t E, const int32_t* conn, const double* Xg, double* dNdX, double* w) {
+// the kT10Grad values of load_g at the 4 quadrature points (SoA) and detJ/24 per element
+__global__ void k_t10_shape(int64_t E, const int32_t* conn, const double* Xg, double* grad, double* w) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= E) return;
-    double X[30], out[30];
+    double X[30], v[4][3], fac;
     for (int k = 0; k < 10; k++) {
         const int64_t n = conn[e * 10 + k];
         for (int c = 0; c < 3; c++) X[3 * k + c] = Xg[3 * n + c];
     }
-    const double qa = (5 + 3 * sqrt(5.0)) / 20, qb = (5 - sqrt(5.0)) / 20;
-    const double L[5][4] = {{qa, qb, qb, qb}, {qb, qa, qb, qb}, {qb, qb, qa, qb}, {qb, qb, qb, qa},
-                            {0.25, 0.25, 0.25, 0.25}};
-    double detJ = 0.0;
-    for (int q = 0; q < 5; q++) {
-        detJ = t10_shape_point(X, L[q][0], L[q][1], L[q][2], L[q][3], out);
-        if (q < 4)
-            for (int r = 0; r < 30; r++) dNdX[(int64_t)(q * 30 + r) * E + e] = out[r];
+    const double qa = t10_qa(), qb = t10_qb();
+    for (int q = 0; q < 4; q++) {
+        t10_shape_vectors(X, q == 0 ? qa : qb, q == 1 ? qa : qb, q == 2 ? qa : qb, q == 3 ? qa : qb, v, fac);
+        double* p = grad + (int64_t)(kT10Grad * q) * E + e;
+        for (int r = 0; r < 12; r++) p[(int64_t)r * E] = v[r / 3][r % 3];
+        p[(int64_t)12 * E] = fac;
     }
-    w[e] = detJ / 24.0;
+    w[e] = t10_shape_vectors(X, 0.25, 0.25, 0.25, 0.25, v, fac) / 24.0;
 }
 
 // Per-element state for export, one thread per element: the passive PK2 stress in
@@ -1235,16 +1357,18 @@ __global__ void __launch_bounds__(128) k_element_export(ElemArgs a, const double
     }
     double F[9];
     if (NPE == 10) {
-        double X[30], dN[30];
+        double X[30], v[4][3], fac, dN[10][3];
         for (int k = 0; k < 10; k++) {
             const int64_t n = a.conn[(int64_t)k * E + e];
             for (int c = 0; c < 3; c++) X[3 * k + c] = Xref[3 * n + c];
         }
-        t10_shape_point(X, 0.25, 0.25, 0.25, 0.25, dN);
+        const double l[4] = {0.25, 0.25, 0.25, 0.25};
+        t10_shape_vectors(X, 0.25, 0.25, 0.25, 0.25, v, fac);
+        for (int k = 0; k < 10; k++) t10_gradient(k, l, v, fac, dN[k]);
         for (int i = 0; i < 3; i++)
             for (int j = 0; j < 3; j++) {
                 double t = 0.0;
-                for (int k = 0; k < 10; k++) t += dN[3 * k + j] * x[3 * k + i];
+                for (int k = 0; k < 10; k++) t += dN[k][j] * x[3 * k + i];
                 F[3 * i + j] = t;
             }
     } else {
@@ -1278,11 +1402,13 @@ void launch_element_residual(int npe, const ElemArgs& a, hipStream_t s) {
     if (a.E == 0) return;
     const int nblk = (int)((a.E + kResidualBlock - 1) / kResidualBlock);
     const bool l17 = a.l17_params != nullptr;
-    if (npe == 10 && l17)
-        hipLaunchKernelGGL((k_residual<10, 4, true>), dim3(nblk, a.n_sets), dim3(kResidualBlock), 0, s, a);
-    else if (npe == 10)
-        hipLaunchKernelGGL((k_residual<10, 4>), dim3(nblk, a.n_sets), dim3(kResidualBlock), 0, s, a);
-    else if (l17)
+    if (npe == 10) {
+        const dim3 grid((unsigned)((a.E + 63) / 64), a.n_sets);
+        if (l17)
+            hipLaunchKernelGGL(k_residual_t10<true>, grid, dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL(k_residual_t10<false>, grid, dim3(256), 0, s, a);
+    } else if (l17)
         hipLaunchKernelGGL((k_residual<4, 1, true>), dim3(nblk, a.n_sets), dim3(kResidualBlock), 0, s, a);
     else
         hipLaunchKernelGGL((k_residual<4, 1>), dim3(nblk, a.n_sets), dim3(kResidualBlock), 0, s, a);
