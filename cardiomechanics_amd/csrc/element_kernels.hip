@@ -827,6 +827,7 @@ __global__ __launch_bounds__(64) void k_residual_tangent(const ElemArgs a0) {
 // gives each (element, i, j) BSPLIT lanes, one per part of the node range b, in a
 // workgroup of BSPLIT waves: fewer accumulators per lane, more waves per SIMD.
 // ---------------------------------------------------------------------------
+constexpr int kCUs = 256;
 constexpr int kQRec = 51;   // Ft(9) BBt(9) S(9) Z(9) Y|X(9) czz codot ceq d00 d11 mfs
 
 // STAGED: the accumulators of the workgroup's elements go through LDS (the quadrature
@@ -1466,8 +1467,20 @@ void launch_element_residual_tangent(int npe, bool fp32, const ElemArgs& a, hipS
             if (fp32) CMG_LAUNCH((k_residual_tangent<4, 1, float>));
             else CMG_LAUNCH((k_residual_tangent<4, 1, double>));
         } else {
-            if (fp32) CMG_LAUNCH((k_residual_tangent_v2<4, 1, float, 1>));
-            else CMG_LAUNCH((k_residual_tangent_v2<4, 1, double, 1>));
+            // T4 has one point per element: with seven elements per workgroup its stage A fills seven
+            // lanes of a wave.  Eight groups fill 56 (FP64 / mixed, us: 24,576 elements 20.4 / 18.0
+            // against 24.3 / 22.7, 200,340 elements 138 / 110 against 160 / 124) where that leaves
+            // a workgroup for every CU; below, more CUs at work count (384 elements 8.4 / 8.6)
+            constexpr int kWide = 8;
+            const int64_t wide = (a.E + kWide * kTanElemsPerWave - 1) / (kWide * kTanElemsPerWave);
+            if (wide * a.n_sets < kCUs) {
+                if (fp32) CMG_LAUNCH((k_residual_tangent_v2<4, 1, float, 1>));
+                else CMG_LAUNCH((k_residual_tangent_v2<4, 1, double, 1>));
+            } else {
+                const dim3 grid((unsigned)wide, a.n_sets), block(64 * kWide);
+                if (fp32) hipLaunchKernelGGL((k_residual_tangent_v2<4, 1, float, 1, 1, kWide>), grid, block, 0, s, a);
+                else hipLaunchKernelGGL((k_residual_tangent_v2<4, 1, double, 1, 1, kWide>), grid, block, 0, s, a);
+            }
         }
     }
 #undef CMG_LAUNCH
