@@ -174,7 +174,7 @@ void cmg_default_options(cmg_options* o) {
     o->krylov_maxit = 4000;
     o->krylov_method = 2;   // BiCGStab
     o->device = 0;
-    o->element_variant = 0;   // by precision: 6 (FP64), 5 (mixed), the fastest of each on the LV
+    o->element_variant = 0;   // 6, the fastest on the LV
     o->newton_atol = 1e-8;
     o->newton_rtol = 1e-8;
     o->newton_stol = 1e-8;
@@ -225,7 +225,7 @@ int cmg_create(const cmg_mesh* mesh, const cmg_material* materials, int32_t n_ma
         cmg_default_options(&c->opt);
     if (c->opt.spmv_choice < 0 || c->opt.spmv_choice > 9) return fail("cmg_options.spmv_choice must be 0-9");
     if (c->opt.element_variant < 1 || c->opt.element_variant > 8)
-        c->opt.element_variant = (c->opt.precision == CMG_PREC_MIXED) ? 5 : 6;
+        c->opt.element_variant = 6;
     if (!std::isfinite(c->opt.rayleigh_alpha) || !std::isfinite(c->opt.rayleigh_beta))
         return fail("cmg_create: Rayleigh damping coefficients must be finite");
     c->device = c->opt.device;

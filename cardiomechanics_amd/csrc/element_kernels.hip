@@ -815,6 +815,59 @@ __global__ __launch_bounds__(64) void k_residual_tangent(const ElemArgs a0) {
     }
 }
 
+// M^{ij}_{mP} of one point from its record (see the file header)
+template <typename TT>
+__device__ __forceinline__ void moduli(const ElemArgs& a, int64_t e, const TT* rec, int ii, int jj, TT* M) {
+    const DevMaterial& m = a.mats[a.matidx ? a.matidx[e] : 0];
+    TT u[3], w[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        u[r] = rec[3 * ii + r];
+        w[r] = rec[3 * jj + r];
+    }
+    const TT bbt = rec[9 + 3 * ii + jj], czz = rec[45], codot = rec[46], ceq = rec[47];
+    const TT d00 = rec[48], d11 = rec[49], mfs = rec[50];
+    const TT *S = rec + 18, *Z = rec + 27, *YX = rec + 36;
+    TT Zu[3], Zw[3], Xu[3], Yw[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++) {
+        Zu[r] = Z[3 * r] * u[0] + Z[3 * r + 1] * u[1] + Z[3 * r + 2] * u[2];
+        Zw[r] = Z[3 * r] * w[0] + Z[3 * r + 1] * w[1] + Z[3 * r + 2] * w[2];
+        Xu[r] = YX[3 * r] * u[0] + YX[3 * r + 1] * u[1] + YX[3 * r + 2] * u[2];
+        Yw[r] = YX[3 * r] * w[0] + YX[3 * r + 1] * w[1] + YX[3 * r + 2] * w[2];
+    }
+    const TT uZw = u[0] * Zw[0] + u[1] * Zw[1] + u[2] * Zw[2];
+#pragma unroll
+    for (int mm = 0; mm < 3; mm++)
+#pragma unroll
+        for (int P = 0; P < 3; P++)
+            M[3 * mm + P] = bbt * S[3 * P + mm] + czz * Zu[mm] * Zw[P] +
+                            codot * (uZw * Z[3 * mm + P] + Zu[P] * Zw[mm]);
+    if (m.law == CMG_LAW_GUCCIONE) {
+        const TT bf = (TT)m.p[1], bt = (TT)m.p[2], bfs = (TT)m.p[3];
+        const TT bmat[9] = {bf, bfs, bfs, bfs, bt, bt, bfs, bt, bt};
+        const TT hc = (TT)0.5 * ceq, oc = (TT)2.0 * ceq;
+        TT h[3];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+            h[r] = u[0] * w[0] * bmat[r] + u[1] * w[1] * bmat[3 + r] + u[2] * w[2] * bmat[6 + r];
+#pragma unroll
+        for (int mm = 0; mm < 3; mm++)
+#pragma unroll
+            for (int P = 0; P < 3; P++)
+                M[3 * mm + P] += hc * (u[P] * w[mm] * bmat[3 * P + mm] + ((mm == P) ? h[mm] : (TT)0)) +
+                                 oc * Xu[mm] * Yw[P];
+    } else {
+        const TT av[3] = {u[1], u[0], (TT)0}, bv[3] = {w[1], w[0], (TT)0};
+#pragma unroll
+        for (int mm = 0; mm < 3; mm++)
+#pragma unroll
+            for (int P = 0; P < 3; P++) M[3 * mm + P] += Xu[mm] * w[P] + mfs * av[mm] * bv[P];
+        M[4] += d11 * u[1] * w[1];
+    }
+    M[0] += d00 * u[0] * w[0];
+}
+
 // ---------------------------------------------------------------------------
 // residual + tangent, shared quadrature-point stage (v2)
 //
@@ -945,15 +998,6 @@ __global__ __launch_bounds__(64 * BSPLIT * GROUPS) void k_residual_tangent_v2(co
     const int b0 = bh * BH;
     TT keep[STAGED ? AH * BH : 1];   // V K_e entries of this lane for the staged store
     if (valid) {
-        const DevMaterial& m = a.mats[a.matidx ? a.matidx[e] : 0];
-        const bool guc = m.law == CMG_LAW_GUCCIONE;
-        TT bmat[9];
-        {
-            const TT bf = (TT)m.p[1], bt = (TT)m.p[2], bfs = (TT)m.p[3];
-            const TT bb[9] = {bf, bfs, bfs, bfs, bt, bt, bfs, bt, bt};
-#pragma unroll
-            for (int r = 0; r < 9; r++) bmat[r] = bb[r];
-        }
         const double V = a.w[e];
         TT* Ke = static_cast<TT*>(a.Ke) + e * (9 * NPE * NPE);
 #pragma unroll 1
@@ -963,58 +1007,8 @@ __global__ __launch_bounds__(64 * BSPLIT * GROUPS) void k_residual_tangent_v2(co
             for (int r = 0; r < AH * BH; r++) acc[r] = (TT)0;
 #pragma unroll 1
             for (int q = 0; q < NQP; q++) {
-                const TT* rec = sQ[slot][q];
-                TT u[3], w[3], Z[9], S[9], YX[9];
-#pragma unroll
-                for (int r = 0; r < 3; r++) {
-                    u[r] = rec[3 * ii + r];
-                    w[r] = rec[3 * jj + r];
-                }
-#pragma unroll
-                for (int r = 0; r < 9; r++) {
-                    S[r] = rec[18 + r];
-                    Z[r] = rec[27 + r];
-                    YX[r] = rec[36 + r];
-                }
-                const TT bbt = rec[9 + ij], czz = rec[45], codot = rec[46], ceq = rec[47];
-                const TT d00 = rec[48], d11 = rec[49], mfs = rec[50];
-                TT Zu[3], Zw[3], Xu[3], Yw[3];
-#pragma unroll
-                for (int r = 0; r < 3; r++) {
-                    Zu[r] = Z[3 * r] * u[0] + Z[3 * r + 1] * u[1] + Z[3 * r + 2] * u[2];
-                    Zw[r] = Z[3 * r] * w[0] + Z[3 * r + 1] * w[1] + Z[3 * r + 2] * w[2];
-                    Xu[r] = YX[3 * r] * u[0] + YX[3 * r + 1] * u[1] + YX[3 * r + 2] * u[2];
-                    Yw[r] = YX[3 * r] * w[0] + YX[3 * r + 1] * w[1] + YX[3 * r + 2] * w[2];
-                }
-                const TT uZw = u[0] * Zw[0] + u[1] * Zw[1] + u[2] * Zw[2];
                 TT M[9];
-#pragma unroll
-                for (int mm = 0; mm < 3; mm++)
-#pragma unroll
-                    for (int P = 0; P < 3; P++)
-                        M[3 * mm + P] = bbt * S[3 * P + mm] + czz * Zu[mm] * Zw[P] +
-                                        codot * (uZw * Z[3 * mm + P] + Zu[P] * Zw[mm]);
-                if (guc) {
-                    const TT hc = (TT)0.5 * ceq, oc = (TT)2.0 * ceq;
-                    TT h[3];
-#pragma unroll
-                    for (int r = 0; r < 3; r++)
-                        h[r] = u[0] * w[0] * bmat[r] + u[1] * w[1] * bmat[3 + r] + u[2] * w[2] * bmat[6 + r];
-#pragma unroll
-                    for (int mm = 0; mm < 3; mm++)
-#pragma unroll
-                        for (int P = 0; P < 3; P++)
-                            M[3 * mm + P] += hc * (u[P] * w[mm] * bmat[3 * P + mm] + ((mm == P) ? h[mm] : (TT)0)) +
-                                             oc * Xu[mm] * Yw[P];
-                } else {
-                    const TT av[3] = {u[1], u[0], (TT)0}, bv[3] = {w[1], w[0], (TT)0};
-#pragma unroll
-                    for (int mm = 0; mm < 3; mm++)
-#pragma unroll
-                        for (int P = 0; P < 3; P++) M[3 * mm + P] += Xu[mm] * w[P] + mfs * av[mm] * bv[P];
-                    M[4] += d11 * u[1] * w[1];
-                }
-                M[0] += d00 * u[0] * w[0];
+                moduli(a, e, sQ[slot][q], ii, jj, M);
                 TT G[NPE][3];
 #pragma unroll
                 for (int k = 0; k < NPE; k++)
@@ -1095,6 +1089,224 @@ __global__ __launch_bounds__(64 * BSPLIT * GROUPS) void k_residual_tangent_v2(co
                 TT* dst = static_cast<TT*>(a.Ke) + (e0 + sl) * (9 * NPE * NPE) + r0 * ROW;
                 reinterpret_cast<uint4*>(dst)[off] = v;
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// T10 residual + tangent in three stages (variant 6 and the default)
+//
+// A workgroup takes 14 elements, with four waves in FP64 and two in mixed precision.
+//   points  56 lanes of the first wave: F, the law, the residual terms and G = B^-1 dN/dX of one
+//           quadrature point each, to LDS.  What is needed again after the law (B, its inverse,
+//           the gradients' 12 numerators) waits in LDS instead of 60 registers.
+//   moduli  M^{ij} of every point and spatial pair (504 tasks), into the space of the terms
+//           they are made from; the element residuals
+//   blocks  lane (element, i, j, part of the nodes b): K(a,b)_ij = sum_q G_a . (M G_b), the
+//           products M G_b held, G_a streamed from LDS; K_e leaves through LDS in 16-byte units
+// Bound by latency in the first stage (one wave, some 1,500 dependent FP64 operations, 8 us)
+// and by K_e's 7,200 bytes per element in the last: 200k elements, FP64, 242 us for the first
+// stage alone, 321 us for the stores alone.  Waves in flight decide: at most 168 registers
+// (F node by node, values parked in LDS, M from LDS) and 50 KB let three workgroups share a CU
+// instead of two.  Against M recomputed by every lane at two waves per SIMD (FP64 / mixed, us):
+// 200k elements 556 / 348 and 613 / 414, 20k 56 / 45 and 63 / 47.6, 5k 23 / 21.5 and 22 / 21.
+// ---------------------------------------------------------------------------
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+constexpr int kRtElems = 2 * kTanElemsPerWave;   // elements per workgroup
+constexpr int kRtPoints = 4 * kRtElems;
+
+template <typename TT, bool LAND17, int HALVES>
+__global__ __launch_bounds__(128 * HALVES, 3) void k_residual_tangent_t10(const ElemArgs a0, bool stream) {
+    constexpr int kThreads = 128 * HALVES, kNodes = 10 / HALVES;   // nodes b of a lane
+    // G; the points' residual terms and records, then M[point][ij][9]; finally kRows node rows
+    // of K_e per element
+    constexpr size_t kG = sizeof(TT) * kRtPoints * 30;
+    constexpr size_t kTerms = sizeof(double) * kRtPoints * 30, kRecords = sizeof(TT) * kRtPoints * kQRec;
+    constexpr int kRows = sizeof(TT) == 8 ? 5 : 4;
+    constexpr size_t kStage = sizeof(TT) * kRtElems * kRows * 90;
+    static_assert(sizeof(TT) * kRtPoints * 81 <= kTerms + kRecords, "the moduli fit into the space of the terms");
+    __shared__ __align__(16) unsigned char smem[kG + kTerms + kRecords > kStage ? kG + kTerms + kRecords : kStage];
+    auto& sT = *reinterpret_cast<double (*)[kRtPoints][30]>(smem);
+    auto& sQ = *reinterpret_cast<TT (*)[kRtPoints][kQRec]>(smem + kTerms);
+    auto& sM = *reinterpret_cast<TT (*)[kRtPoints][81]>(smem);
+    auto& sG = *reinterpret_cast<TT (*)[kRtPoints][30]>(smem + kTerms + kRecords);
+    auto& stage = *reinterpret_cast<TT (*)[kRtElems][kRows][90]>(smem);
+    ElemArgs a;
+    if (!batch_select(a0, a)) return;
+    const int t = threadIdx.x;
+    const int64_t E = a.E, e0 = (int64_t)xcd_swizzle(blockIdx.x, gridDim.x) * kRtElems;
+    // ---- points ----
+    if (t < kRtPoints && e0 + t % kRtElems < E) {
+        const int q = t / kRtElems, slot = t - kRtElems * q;   // consecutive lanes, consecutive elements
+        const int pt = 4 * slot + q;
+        const int64_t e = e0 + slot;
+        const DevMaterial& m = a.mats[a.matidx ? a.matidx[e] : 0];
+        double ts;
+        const double Ta = tension_of(m, a.time, a.tact[e], ts);
+        L17 l17s;
+        const L17* l17 = nullptr;
+        if (LAND17 && m.tension_fn == CMG_FN_LAND17) {
+            load_l17(a, e, a.matidx ? a.matidx[e] : 0, m, l17s);
+            l17 = &l17s;
+        }
+        double l[4], fac, Floc[9];
+        double* park = sT[pt];
+        {
+            double v[4][3], F[9], B[9], Binv[9];
+            fac = load_t10(a, e, q, l, v);
+#pragma unroll
+            for (int r = 0; r < 9; r++) B[r] = a.bases[(int64_t)(q * 9 + r) * E + e];
+            t10_F(a, e, l, v, fac, F);
+            to_fibre_frame(F, B, Binv, Floc);
+#pragma unroll
+            for (int r = 0; r < 9; r++) {
+                park[r] = B[r];
+                park[9 + r] = Binv[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 12; r++) park[18 + r] = v[r / 3][r % 3];
+        }
+        Law L;
+        if (!eval_law(m, Floc, Ta, ts, true, L, l17)) atomicMin(a.corrupt, (int)e);
+        // the parked values, through an index that the compiler cannot follow back to them
+        int same = pt;
+        asm volatile("" : "+v"(same));
+        double B[9], Binv[9];
+#pragma unroll
+        for (int r = 0; r < 9; r++) {
+            B[r] = sT[same][r];
+            Binv[r] = sT[same][9 + r];
+        }
+        TT* rec = sQ[pt];
+        {
+            double Ft[9];
+            mul3(B, Floc, Ft);
+#pragma unroll
+            for (int r = 0; r < 9; r++) {
+                rec[r] = (TT)Ft[r];
+                rec[9 + r] = (TT)(B[3 * (r / 3)] * B[3 * (r % 3)] + B[3 * (r / 3) + 1] * B[3 * (r % 3) + 1] +
+                                  B[3 * (r / 3) + 2] * B[3 * (r % 3) + 2]);
+                rec[18 + r] = (TT)L.S[r];
+                rec[27 + r] = (TT)L.Z[r];
+                rec[36 + r] = (TT)((m.law == CMG_LAW_GUCCIONE) ? L.Y[r] : L.X[r]);
+            }
+            rec[45] = (TT)L.czz;
+            rec[46] = (TT)L.codot;
+            rec[47] = (TT)((m.law == CMG_LAW_GUCCIONE) ? L.ceq : 0.0);
+            rec[48] = (TT)L.d00;
+            rec[49] = (TT)L.d11;
+            rec[50] = (TT)L.mfs;
+        }
+        double P[9];
+        {
+#pragma clang fp contract(off)
+            double FS[9], St[9], BinvT[9], Bt[9], P1[9];
+            mul3(Floc, L.S, FS);
+            tr3(FS, St);
+            tr3(Binv, BinvT);
+            tr3(B, Bt);
+            mul3(BinvT, St, P1);
+            mul3(P1, Bt, P);
+        }
+        double v[4][3];
+#pragma unroll
+        for (int r = 0; r < 12; r++) v[r / 3][r % 3] = sT[same][18 + r];
+#pragma unroll
+        for (int k = 0; k < 10; k++) {
+            double g[3];
+            t10_gradient(k, l, v, fac, g);
+            {
+#pragma clang fp contract(off)
+#pragma unroll
+                for (int c = 0; c < 3; c++) sT[pt][3 * k + c] = g[0] * P[0 + c] + g[1] * P[3 + c] + g[2] * P[6 + c];
+            }
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+                sG[pt][3 * k + r] = (TT)(Binv[3 * r] * g[0] + Binv[3 * r + 1] * g[1] + Binv[3 * r + 2] * g[2]);
+        }
+    }
+    __syncthreads();
+    // ---- moduli, residuals ----
+    const int nel = (int)(E - e0 < kRtElems ? E - e0 : kRtElems);
+    constexpr int kTasks = (9 * kRtPoints + kThreads - 1) / kThreads;
+    TT M[kTasks][9];
+#pragma unroll
+    for (int k = 0; k < kTasks; k++) {
+        const int pt = (t + kThreads * k) / 9, ij = t + kThreads * k - 9 * pt;
+        if (pt < 4 * nel) moduli(a, e0 + pt / 4, sQ[pt], ij / 3, ij % 3, M[k]);
+    }
+    for (int k = t; k < 30 * nel; k += kThreads) {
+        const int slot = k / 30, r = k - 30 * slot;
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) s += sT[4 * slot + q][r];
+        a.fe[30 * e0 + k] = a.w[e0 + slot] * s;
+    }
+    __syncthreads();   // the terms are consumed
+#pragma unroll
+    for (int k = 0; k < kTasks; k++) {
+        const int pt = (t + kThreads * k) / 9, ij = t + kThreads * k - 9 * pt;
+        if (pt < 4 * nel)
+#pragma unroll
+            for (int r = 0; r < 9; r++) sM[pt][9 * ij + r] = M[k][r];
+    }
+    __syncthreads();
+    // ---- blocks: wave HALVES g + h takes the elements 7 g .. 7 g + 6 and kNodes nodes b ----
+    const int lane = t % 64, h = HALVES == 1 ? 0 : (t / 64) % 2;
+    const int slot = kTanElemsPerWave * (t / (64 * HALVES)) + lane / 9, ij = lane % 9;
+    const bool valid = lane < 9 * kTanElemsPerWave && slot < nel;
+    TT acc[10][kNodes];
+#pragma unroll
+    for (int aa = 0; aa < 10; aa++)
+#pragma unroll
+        for (int b = 0; b < kNodes; b++) acc[aa][b] = (TT)0;
+    if (valid)
+#pragma unroll 1
+    for (int q = 0; q < 4; q++) {
+        const TT* Mp = sM[4 * slot + q] + 9 * ij;
+        const TT* G = sG[4 * slot + q];
+        TT mg[kNodes][3];
+        {
+            TT mm[9];
+#pragma unroll
+            for (int r = 0; r < 9; r++) mm[r] = Mp[r];
+#pragma unroll
+            for (int b = 0; b < kNodes; b++) {
+                const TT *gb = G + 3 * kNodes * h + 3 * b, g0 = gb[0], g1 = gb[1], g2 = gb[2];
+#pragma unroll
+                for (int r = 0; r < 3; r++) mg[b][r] = mm[3 * r] * g0 + mm[3 * r + 1] * g1 + mm[3 * r + 2] * g2;
+            }
+        }
+#pragma unroll
+        for (int aa = 0; aa < 10; aa++) {
+            const TT g0 = G[3 * aa], g1 = G[3 * aa + 1], g2 = G[3 * aa + 2];
+#pragma unroll
+            for (int b = 0; b < kNodes; b++)
+                acc[aa][b] = fma(g2, mg[b][2], fma(g1, mg[b][1], fma(g0, mg[b][0], acc[aa][b])));
+        }
+    }
+    // the blocks leave through LDS, kRows rows of every element at a time, in 16-byte units
+    const TT V = valid ? (TT)a.w[e0 + slot] : (TT)0;
+    static_assert(2 * 90 * sizeof(TT) % 16 == 0 && (sizeof(TT) == 8 || kRows % 2 == 0), "16-byte runs");
+#pragma unroll
+    for (int r0 = 0; r0 < 10; r0 += kRows) {
+        __syncthreads();   // M and G, or the rows before, are consumed
+        const int rows = 10 - r0 < kRows ? 10 - r0 : kRows, units = rows * 90 * (int)sizeof(TT) / 16;
+        if (valid)
+#pragma unroll
+            for (int aa = 0; aa < rows; aa++)
+#pragma unroll
+                for (int b = 0; b < kNodes; b++) stage[slot][aa][9 * (kNodes * h + b) + ij] = V * acc[r0 + aa][b];
+        __syncthreads();
+        for (int u = t; u < nel * units; u += kThreads) {
+            const int el = u / units, off = u - el * units;
+            TT* row = static_cast<TT*>(a.Ke) + (e0 + el) * 900 + 90 * r0;
+            f64x2* dst = reinterpret_cast<f64x2*>(row) + off;
+            const f64x2 v = reinterpret_cast<const f64x2*>(&stage[el][0][0])[off];
+            if (stream)
+                __builtin_nontemporal_store(v, dst);
+            else
+                *dst = v;
         }
     }
 }
@@ -1429,11 +1641,17 @@ void launch_element_residual_tangent(int npe, bool fp32, const ElemArgs& a, hipS
     const int nblk2 = (int)((a.E + 2 * kTanElemsPerWave - 1) / (2 * kTanElemsPerWave));
 #define CMG_LAUNCH(K) hipLaunchKernelGGL(K, dim3(nblk, a.n_sets), dim3(64), 0, s, a)
 #define CMG_LAUNCH2(K) hipLaunchKernelGGL(K, dim3(nblk, a.n_sets), dim3(128), 0, s, a)
+// K_e larger than the 256 MB of the memory-side cache passes it by: the gather reads it from
+// memory anyway (200k elements 556 / 577 us in FP64, 348 / 369 mixed; 20k, which stay in it,
+// 59 / 56 and 47.8 / 45.0)
+#define CMG_LAUNCH_T10(TT, L17, HALVES)                                                                            \
+    hipLaunchKernelGGL((k_residual_tangent_t10<TT, L17, HALVES>), dim3(nblk2, a.n_sets), dim3(128 * HALVES), 0, s, a, \
+                       (size_t)a.E * a.n_sets * 900 * sizeof(TT) > (size_t)256 << 20)
 #define CMG_LAUNCH_G2(K, T) hipLaunchKernelGGL(K, dim3(nblk2, a.n_sets), dim3(T), 0, s, a)
     if (a.l17_params) {
         // Land17 contexts: one shape per element type (the tuned variants stay free of its code)
-        if (npe == 10 && fp32) CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, float, 1, 2, 2, true>), 256);
-        else if (npe == 10) CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, double, 1, 2, 2, true>), 256);
+        if (npe == 10 && fp32) CMG_LAUNCH_T10(float, true, 1);
+        else if (npe == 10) CMG_LAUNCH_T10(double, true, 2);
         else if (fp32) CMG_LAUNCH((k_residual_tangent_v2<4, 1, float, 1, 1, 1, true>));
         else CMG_LAUNCH((k_residual_tangent_v2<4, 1, double, 1, 1, 1, true>));
     } else if (npe == 10) {
@@ -1441,8 +1659,8 @@ void launch_element_residual_tangent(int npe, bool fp32, const ElemArgs& a, hipS
             if (fp32) CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, float, 1, 1, 2>), 128);
             else CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, double, 1, 1, 2>), 128);
         } else if (variant == 6) {
-            if (fp32) CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, float, 1, 2, 2>), 256);
-            else CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, double, 1, 2, 2>), 256);
+            if (fp32) CMG_LAUNCH_T10(float, false, 1);
+            else CMG_LAUNCH_T10(double, false, 2);
         } else if (variant == 7) {
             if (fp32) CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, float, 1, 2, 2, false, true>), 256);
             else CMG_LAUNCH_G2((k_residual_tangent_v2<10, 4, double, 1, 2, 2, false, true>), 256);
@@ -1486,6 +1704,7 @@ void launch_element_residual_tangent(int npe, bool fp32, const ElemArgs& a, hipS
 #undef CMG_LAUNCH
 #undef CMG_LAUNCH2
 #undef CMG_LAUNCH_G2
+#undef CMG_LAUNCH_T10
 }
 
 void launch_surface(const SurfArgs& a, bool tangent, hipStream_t s) {

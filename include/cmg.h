@@ -122,11 +122,12 @@ typedef struct cmg_options {
     int32_t device;             /* HIP device ordinal (default 0) */
     int32_t element_variant;    /* residual+tangent kernel: 2 shared quadrature stage, 3 the same in
                                    two node passes, 4 the same with two lanes per element and
-                                   spatial pair, 1 per-lane quadrature points, 5 / 6 variants 2 / 4
-                                   with 14 elements per workgroup, 7 / 8 variants 6 / 5 with the
-                                   element tangents written through LDS as contiguous 16-byte
-                                   runs; 0 (default): 6 in FP64, 5 in mixed precision.  A context
-                                   with a Land17 material always runs the shape of variant 6 */
+                                   spatial pair, 1 per-lane quadrature points, 5 variant 2 with 14
+                                   elements per workgroup, 6 points, moduli and blocks in three
+                                   stages, 14 elements per workgroup (T10), 7 / 8 variants 4 / 5
+                                   with 14 elements and the element tangents written through LDS
+                                   as contiguous 16-byte runs; 0 (default): 6.  A context with a
+                                   Land17 material always runs the shape of variant 6 */
     int32_t krylov_method;      /* 0 GMRES(restart), 1 or 2 (default) BiCGStab with device-side scalars and
                                    graph-replayed iterations (one solver, two accepted names); right
                                    preconditioned (see preconditioner) */
