@@ -8,10 +8,18 @@
 //   matrix: each 3x3 block sums the element/surface blocks that map to it, adds
 //           cm * M (mass stored as one scalar per block) and puts the identity on
 //           constrained DOFs (CBSolver.cpp:413-435, :323-324).
+#include <climits>
+
 #include "cmg_internal.h"
 
 namespace cmg {
 namespace {
+
+__device__ __forceinline__ void publish(const SetStrides& b, int flag) {
+    __hip_atomic_store(b.word, flag_word(b.seq, flag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void k_publish_flag(SetStrides b) { publish(b, *b.corrupt); }
 
 __global__ __launch_bounds__(256) void k_gather_vector(int64_t N, const int64_t* inc_ptr, const int32_t* inc,
                                                        const double* fe, const int64_t* sinc_ptr,
@@ -19,6 +27,11 @@ __global__ __launch_bounds__(256) void k_gather_vector(int64_t N, const int64_t*
                                                        const uint8_t* bcmask, double* f, SetStrides b) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t set = blockIdx.y;
+    if (b.corrupt) {
+        const int flag = *b.corrupt;
+        if (b.word && blockIdx.x == 0 && threadIdx.x == 0) publish(b, flag);
+        if (flag != INT_MAX) return;
+    }
     if (r >= N || (b.active && !b.active[set])) return;
     fe += set * b.a;
     if (fs) fs += set * b.b;
@@ -136,6 +149,7 @@ __global__ __launch_bounds__(256) void k_gather_matrix(int64_t nnzb, const int64
                                                        VT* vals, bool flip, SetStrides st) {
     const int64_t set = blockIdx.y;
     if (st.active && !st.active[set]) return;
+    if (st.corrupt && *st.corrupt != INT_MAX) return;
     // (workgroups in plain order: giving each XCD a contiguous range of slots measured
     // 19 % slower on the 200k-element LV, with the same HBM fetch)
     int64_t slot;
@@ -199,6 +213,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(GatherMaps g, co
     extern __shared__ double row_acc[];   // [kRowWaves][row_cap * 9]
     const int64_t set = blockIdx.y;
     if (st.active && !st.active[set]) return;
+    if (st.corrupt && *st.corrupt != INT_MAX) return;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int l = (int)(threadIdx.x & 63);
     const int64_t r = (int64_t)blockIdx.x * kRowWaves + w;
@@ -357,6 +372,10 @@ void launch_add_scaled_values(int64_t nnzb, double a, const double* C, void* val
         hipLaunchKernelGGL(k_add_scaled_values<float>, grid, dim3(256), 0, s, nv, a, C, (float*)vals);
     else
         hipLaunchKernelGGL(k_add_scaled_values<double>, grid, dim3(256), 0, s, nv, a, C, (double*)vals);
+}
+
+void launch_publish_flag(const SetStrides& b, hipStream_t s) {
+    hipLaunchKernelGGL(k_publish_flag, dim3(1), dim3(1), 0, s, b);
 }
 
 void launch_gather_vector(int64_t N, const int64_t* inc_ptr, const int32_t* inc, const double* fe, int,

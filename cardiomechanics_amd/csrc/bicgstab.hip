@@ -411,20 +411,7 @@ int wait_for(cmg_ctx* c, unsigned seq, int it, unsigned long long& word) {
         word = __atomic_load_n(w, __ATOMIC_ACQUIRE);
         return (unsigned)(word >> 40) == seq && ((int)((word >> 8) & 0xffffffffu) >= it || (word & 0xff) != 0);
     };
-    for (unsigned spin = 1;; spin++) {
-        if (reached()) return CMG_SUCCESS;
-        if (spin % 2048 == 0) {
-            const hipError_t e = hipStreamQuery(c->stream);
-            if (e == hipErrorNotReady) {
-                (void)hipGetLastError();
-                continue;
-            }
-            CMG_HIP_CHECK(e);
-            if (reached()) return CMG_SUCCESS;
-            return fail("BiCGStab: the stream has drained without the expected iteration", CMG_ERR_HIP);
-        }
-        __builtin_ia32_pause();
-    }
+    return wait_host(c, reached);
 }
 
 }  // namespace

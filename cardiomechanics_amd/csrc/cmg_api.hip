@@ -202,6 +202,7 @@ void cmg_destroy(cmg_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->bicg_graph) (void)hipGraphExecDestroy(c->bicg_graph);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
+    if (c->flag_host) (void)hipHostFree(c->flag_host);
     if (c->bicg_host) (void)hipHostFree(c->bicg_host);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -516,7 +517,11 @@ int cmg_create(const cmg_mesh* mesh, const cmg_material* materials, int32_t n_ma
         CMG_TRY(alloc(c->cvals, (size_t)(nnzb + kSpmvPadBlocks) * 9 * sizeof(double)));
         launch_fill((nnzb + kSpmvPadBlocks) * 9, 0.0, c->cvals.as<double>(), s);
     }
-    CMG_TRY(alloc(c->corrupt, sizeof(int)));
+    CMG_TRY(alloc(c->corrupt, 2 * sizeof(int)));
+    launch_fill_int(2, INT_MAX, c->corrupt.as<int>(), s);
+    CMG_HIP_CHECK(hipHostMalloc((void**)&c->flag_host, sizeof(unsigned long long),
+                                hipHostMallocCoherent | hipHostMallocMapped));
+    *c->flag_host = 0;
     c->gm_m = std::max(8, std::min(c->opt.krylov_restart, 1000));
     CMG_TRY(alloc(c->gm_V, (size_t)(c->gm_m + 2) * vb));
     CMG_TRY(alloc(c->gm_partial, (size_t)dot_blocks(c->n) * (c->gm_m + 2) * sizeof(double) + 64));
@@ -637,11 +642,26 @@ SurfArgs surf_args(cmg_ctx* c, const double* x_dev, bool with_volume) {
 
 namespace {
 
-// element kernels (+ surfaces) at x_dev; returns CMG_SUCCESS or CMG_CORRUPT_ELEMENT
+// the flag of the evaluation in flight, for the gathers queued behind it
+SetStrides eval_flag(cmg_ctx* c, bool publish) {
+    SetStrides b;
+    b.corrupt = c->corrupt.as<int>();
+    b.word = publish ? c->flag_host : nullptr;
+    b.seq = c->flag_seq;
+    return b;
+}
+
+// element kernels (+ surfaces) at x_dev and behind them gather(), which queues the evaluation's
+// gathers (they leave their outputs alone if an element is corrupt) and has the flag published;
+// returns CMG_SUCCESS or CMG_CORRUPT_ELEMENT as soon as the flag is known, with the gathers
+// in flight.  The flag is INT_MAX between evaluations, so none clears it first, and it comes
+// by a word in pinned memory: a fill, a copy and a wait less per evaluation, and the GPU
+// does not stand still between the element kernels and the gathers (residual of the
+// 1,296-element cube 18.7 / 28.8 us, assembly of 24,576 T4 elements 37.7 / 46.7 us).
+template <typename F>
 int eval_elements(cmg_ctx* c, const double* x_dev, double time, bool tangent, bool pressure, int* corrupt_id,
-                  bool fp64_tangent = false) {
+                  bool fp64_tangent, F gather) {
     hipStream_t s = c->stream;
-    launch_fill_int(1, INT_MAX, c->corrupt.as<int>(), s);
     ElemArgs a = elem_args(c, x_dev, time);
     if (tangent && fp64_tangent)
         launch_element_residual_tangent(c->npe, false, a, s, 6);
@@ -650,13 +670,18 @@ int eval_elements(cmg_ctx* c, const double* x_dev, double time, bool tangent, bo
     else
         launch_element_residual(c->npe, a, s);
     if (pressure && c->S > 0) launch_surface(surf_args(c, x_dev, false), tangent && c->opt.pressure_tangent, s);
+    c->flag_seq++;
+    gather();
     CMG_HIP_CHECK(hipGetLastError());
-    int flag = INT_MAX;
-    CMG_HIP_CHECK(hipMemcpyAsync(c->h_pinned, c->corrupt.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    CMG_HIP_CHECK(hipStreamSynchronize(s));
-    std::memcpy(&flag, c->h_pinned, sizeof(int));
+    unsigned long long word = 0;
+    CMG_TRY(wait_host(c, [&]() {
+        word = __atomic_load_n(c->flag_host, __ATOMIC_ACQUIRE);
+        return (unsigned)(word >> 32) == c->flag_seq;
+    }));
+    const int flag = (int)(unsigned)word;
     if (corrupt_id) *corrupt_id = (flag == INT_MAX) ? -1 : flag;
     if (flag != INT_MAX) {
+        launch_fill_int(1, INT_MAX, c->corrupt.as<int>(), s);
         set_error("element " + std::to_string(flag) + " is corrupt (det F <= 0)");
         return CMG_CORRUPT_ELEMENT;
     }
@@ -667,7 +692,8 @@ void gather_residual(cmg_ctx* c, bool pressure, double* f_dev) {
     const bool sp = pressure && c->S > 0;
     launch_gather_vector(c->N, c->inc_ptr.as<int64_t>(), c->inc.as<int32_t>(), c->fe.as<double>(), 3 * c->npe,
                          sp ? c->sinc_ptr.as<int64_t>() : nullptr, sp ? c->sinc.as<int32_t>() : nullptr,
-                         sp ? c->fs.as<double>() : nullptr, 3 * c->nps, c->bcmask.as<uint8_t>(), f_dev, c->stream);
+                         sp ? c->fs.as<double>() : nullptr, 3 * c->nps, c->bcmask.as<uint8_t>(), f_dev, c->stream,
+                         eval_flag(c, true));
 }
 
 void gather_tangent(cmg_ctx* c, bool pressure, double cm, void* vals_dev) {
@@ -675,8 +701,10 @@ void gather_tangent(cmg_ctx* c, bool pressure, double cm, void* vals_dev) {
     // without a pressure tangent the surface blocks read zeros: clear Ks
     if (c->S > 0 && !sp) launch_fill((int64_t)c->S * 9 * c->nps * c->nps, 0.0, c->Ks.as<double>(), c->stream);
     launch_gather_matrix(gather_maps(c), c->Ke.p, c->fp32, c->Ks.as<double>(), cm != 0.0 ? c->mval.as<double>() : nullptr,
-                         cm, c->bcmask.as<uint8_t>(), vals_dev, c->fp32, false, c->stream);
+                         cm, c->bcmask.as<uint8_t>(), vals_dev, c->fp32, false, c->stream, eval_flag(c, false));
 }
+
+void publish_flag(cmg_ctx* c) { launch_publish_flag(eval_flag(c, true), c->stream); }
 
 // ||v||_2 (synchronising)
 int norm2(cmg_ctx* c, const double* v, double* out) {
@@ -947,28 +975,27 @@ extern "C" {
 int cmg_residual_device(cmg_ctx* c, const double* x_dev, double time, int32_t include_pressure, double* f_dev) {
     if (!c || !x_dev || !f_dev) return fail("cmg_residual_device: null argument");
     CMG_HIP_CHECK(hipSetDevice(c->device));
-    int rc = eval_elements(c, x_dev, time, false, include_pressure != 0, nullptr);
-    if (rc != CMG_SUCCESS) return rc;
-    gather_residual(c, include_pressure != 0, f_dev);
-    CMG_HIP_CHECK(hipGetLastError());
-    return CMG_SUCCESS;
+    return eval_elements(c, x_dev, time, false, include_pressure != 0, nullptr, false,
+                         [&]() { gather_residual(c, include_pressure != 0, f_dev); });
 }
 
 int cmg_residual_tangent_device(cmg_ctx* c, const double* x_dev, double time, int32_t include_pressure, double* f_dev,
                                 void* values_dev) {
     if (!c || !x_dev) return fail("cmg_residual_tangent_device: null argument");
     CMG_HIP_CHECK(hipSetDevice(c->device));
-    int rc = eval_elements(c, x_dev, time, true, include_pressure != 0, nullptr);
-    if (rc != CMG_SUCCESS) return rc;
-    if (f_dev) gather_residual(c, include_pressure != 0, f_dev);
-    if (values_dev) gather_tangent(c, include_pressure != 0, 0.0, values_dev);
-    CMG_HIP_CHECK(hipGetLastError());
-    return CMG_SUCCESS;
+    return eval_elements(c, x_dev, time, true, include_pressure != 0, nullptr, false, [&]() {
+        if (f_dev)
+            gather_residual(c, include_pressure != 0, f_dev);
+        else
+            publish_flag(c);
+        if (values_dev) gather_tangent(c, include_pressure != 0, 0.0, values_dev);
+    });
 }
 
 int cmg_element_kernel_device(cmg_ctx* c, const double* x_dev, double time, int32_t with_tangent) {
     if (!c || !x_dev) return fail("cmg_element_kernel_device: null argument");
     ElemArgs a = elem_args(c, x_dev, time);
+    a.corrupt = c->corrupt.as<int>() + 1;   // nobody reads this call's flag
     if (with_tangent)
         launch_element_residual_tangent(c->npe, c->fp32, a, c->stream, c->opt.element_variant);
     else
@@ -1012,7 +1039,7 @@ int cmg_element_residuals(cmg_ctx* c, const double* x, double time, double* fe) 
     if (!c || !x || !fe) return fail("cmg_element_residuals: null argument");
     CMG_HIP_CHECK(hipSetDevice(c->device));
     CMG_HIP_CHECK(hipMemcpyAsync(c->xeval.p, x, c->n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    int rc = eval_elements(c, c->xeval.as<double>(), time, false, false, nullptr);
+    int rc = eval_elements(c, c->xeval.as<double>(), time, false, false, nullptr, false, [&]() { publish_flag(c); });
     if (rc != CMG_SUCCESS) return rc;
     CMG_HIP_CHECK(hipMemcpyAsync(fe, c->fe.p, (size_t)c->E * 3 * c->npe * sizeof(double), hipMemcpyDeviceToHost,
                                  c->stream));
@@ -1024,7 +1051,7 @@ int cmg_element_tangents(cmg_ctx* c, const double* x, double time, void* Ke) {
     if (!c || !x || !Ke) return fail("cmg_element_tangents: null argument");
     CMG_HIP_CHECK(hipSetDevice(c->device));
     CMG_HIP_CHECK(hipMemcpyAsync(c->xeval.p, x, c->n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    int rc = eval_elements(c, c->xeval.as<double>(), time, true, false, nullptr);
+    int rc = eval_elements(c, c->xeval.as<double>(), time, true, false, nullptr, false, [&]() { publish_flag(c); });
     if (rc != CMG_SUCCESS) return rc;
     const int npe = c->npe, nd = 3 * npe;
     const size_t es = c->fp32 ? sizeof(float) : sizeof(double);
@@ -1208,7 +1235,8 @@ int build_damping(cmg_ctx* c, double time) {
     hipStream_t s = c->stream;
     if (c->opt.rayleigh_beta != 0.0) {
         int corrupt = -1;
-        const int rc = eval_elements(c, c->nodes.as<double>(), time, true, false, &corrupt, true);
+        const int rc = eval_elements(c, c->nodes.as<double>(), time, true, false, &corrupt, true,
+                                     [&]() { publish_flag(c); });
         if (rc != CMG_SUCCESS) return rc;
         if (c->S > 0) launch_fill((int64_t)c->S * 9 * c->nps * c->nps, 0.0, c->Ks.as<double>(), s);
         // C is built from the tangent in the reference's layout: for T10 its finite-difference
@@ -1244,11 +1272,11 @@ int residual_norm_at(cmg_ctx* c, double time, double cm, double cd, double* out)
     hipStream_t s = c->stream;
     launch_waxpby(c->n, 1.0, c->nodes.as<double>(), 1.0, c->d.as<double>(), c->xeval.as<double>(), s);
     int corrupt = -1;
-    if (eval_elements(c, c->xeval.as<double>(), time, false, true, &corrupt) != CMG_SUCCESS) {
+    if (eval_elements(c, c->xeval.as<double>(), time, false, true, &corrupt, false,
+                      [&]() { gather_residual(c, true, c->r.as<double>()); }) != CMG_SUCCESS) {
         *out = INFINITY;
         return CMG_SUCCESS;
     }
-    gather_residual(c, true, c->r.as<double>());
     if (cm != 0.0)
         launch_add_mass_term(c->N, c->rowptr.as<int64_t>(), c->colind.as<int32_t>(), c->mval.as<double>(), cm,
                              c->d.as<double>(), c->dpred.as<double>(), c->bcmask.as<uint8_t>(), c->r.as<double>(), s);
@@ -1288,7 +1316,7 @@ int newton(cmg_ctx* c, double time, double cm, double cd, cmg_step_stats* st) {
         int corrupt = -1;
         // residual only: the tangent is evaluated below once the iterate is accepted and a
         // linear solve follows (not at the converged iterate, not on a backtracked one)
-        int rc = eval_elements(c, xe, time, false, true, &corrupt);
+        int rc = eval_elements(c, xe, time, false, true, &corrupt, false, [&]() { gather_residual(c, true, r); });
         if (rc != CMG_SUCCESS) {
             st->corrupt_element = corrupt;
             if (c->trace) std::fprintf(stderr, "[newton]   element %d inverted at lambda=%.4g\n", corrupt, lambda);
@@ -1313,7 +1341,6 @@ int newton(cmg_ctx* c, double time, double cm, double cd, cmg_step_stats* st) {
             st->krylov_iterations = kry_total;
             return CMG_FAILED;
         }
-        gather_residual(c, true, r);
         if (cm != 0.0)
             launch_add_mass_term(c->N, c->rowptr.as<int64_t>(), c->colind.as<int32_t>(), c->mval.as<double>(), cm, d,
                                  c->dpred.as<double>(), c->bcmask.as<uint8_t>(), r, s);
@@ -1380,13 +1407,15 @@ int newton(cmg_ctx* c, double time, double cm, double cd, cmg_step_stats* st) {
             std::min(eta_max, std::max(eta, 0.5 * (c->opt.newton_atol + c->opt.newton_rtol * r0) / rnorm));
         rprev = rnorm;
         const double tb = now_s();
-        rc = eval_elements(c, xe, time, true, true, &corrupt);
+        rc = eval_elements(c, xe, time, true, true, &corrupt, false, [&]() {
+            publish_flag(c);
+            gather_tangent(c, true, cm, c->vals.p);
+        });
         if (rc != CMG_SUCCESS) {   // the residual kernel accepted this state: not expected
             st->corrupt_element = corrupt;
             st->converged_reason = -6;
             break;
         }
-        gather_tangent(c, true, cm, c->vals.p);
         if (cd != 0.0 && c->damping) launch_add_scaled_values(c->nnzb, cd, c->cvals.as<double>(), c->vals.p, c->fp32, s);
         t_tan += now_s() - tb;
         const double tk = now_s();

@@ -137,7 +137,11 @@ struct cmg_ctx {
     cmg::DevBuf gm_V, gm_partial, gm_h, gm_y;
     int gm_m = 0;
     double* h_pinned = nullptr;   // host staging for reductions
+    // corrupt: the element kernels' flag, INT_MAX between evaluations; flag_host: the pinned word
+    // that reports it, with the evaluation's number
     cmg::DevBuf corrupt;
+    unsigned long long* flag_host = nullptr;
+    unsigned flag_seq = 0;
     // static solver bookkeeping (CBSolverEquilibrium::UpdateInitialGuess)
     double time_last = 0.0, step_last = 0.0;
     cmg::DevBuf guess;               // normalised previous increment
@@ -209,4 +213,22 @@ void launch_patch_apply_s(cmg_ctx* c, const BicgVec& k, const double* part, int 
 // zero_guess: x starts at zero whatever it holds
 int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero_guess, double rtol, int maxit,
              cmg_solve_stats* st);
+// polls pinned host memory until reached(), which a kernel queued on the context's stream sees to
+template <typename F>
+int wait_host(cmg_ctx* c, F reached) {
+    for (unsigned spin = 1;; spin++) {
+        if (reached()) return CMG_SUCCESS;
+        if (spin % 2048 == 0) {
+            const hipError_t e = hipStreamQuery(c->stream);
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();
+                continue;
+            }
+            CMG_HIP_CHECK(e);
+            if (reached()) return CMG_SUCCESS;
+            return fail("the stream has drained without the expected report", CMG_ERR_HIP);
+        }
+        __builtin_ia32_pause();
+    }
+}
 }  // namespace cmg

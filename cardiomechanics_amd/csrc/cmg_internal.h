@@ -114,7 +114,17 @@ struct SetStrides {
     int n_sets = 1;
     int64_t a = 0, b = 0, c = 0;   // per-set strides of the kernel's arrays, in elements
     const int32_t* active = nullptr;
+    // a single evaluation's element flag (ElemArgs::corrupt): the outputs stay as they are when an
+    // element is corrupt; word: pinned host memory that the vector gather tells (flag_word)
+    const int* corrupt = nullptr;
+    unsigned long long* word = nullptr;
+    unsigned seq = 0;
 };
+__host__ __device__ inline unsigned long long flag_word(unsigned seq, int flag) {
+    return ((unsigned long long)seq << 32) | (unsigned)flag;
+}
+// the flag alone (evaluations without a vector gather)
+void launch_publish_flag(const SetStrides& b, hipStream_t s);
 void launch_gather_vector(int64_t N, const int64_t* inc_ptr, const int32_t* inc, const double* fe, int stride_e,
                           const int64_t* sinc_ptr, const int32_t* sinc, const double* fs, int stride_s,
                           const uint8_t* bcmask, double* f, hipStream_t s, const SetStrides& b = SetStrides());
