@@ -36,10 +36,14 @@ __device__ __forceinline__ void bicg_publish(const BicgScalars* sc, BicgHost* ho
     __hip_atomic_store(&host->word, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// alpha = rho / (r^, v) from nb <= 256 partials, in every workgroup of 256 threads; the first
-// one stores it, or ends the solve when the product is zero or not finite (false everywhere)
+constexpr int kBicgPartials = 1024;   // partial sums that their consumers add up themselves
+
+// alpha = rho / (r^, v) from nb <= kBicgPartials partials, in every workgroup of 256 threads; the
+// first one stores it, or ends the solve when the product is zero or not finite (false everywhere)
 __device__ __forceinline__ bool bicg_alpha(const BicgVec& k, const double* part, int nb, double* sh, double& alpha) {
-    double d = (int)threadIdx.x < nb ? part[threadIdx.x] : 0.0;
+    double d = 0.0;
+#pragma unroll
+    for (int j = 0; j < kBicgPartials; j += 256) d += j + (int)threadIdx.x < nb ? part[j + threadIdx.x] : 0.0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
     if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = d;

@@ -207,7 +207,7 @@ void launch_coarse_solve(cmg_ctx* c, const PatchSets& ps);
 void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps = PatchSets());  // patch inverses
 // z = sum_p R_p^T A_p^-1 R_p r
 void launch_patch_apply(cmg_ctx* c, const double* r, double* z, const PatchSets& ps = PatchSets());
-// the same for s = r - alpha v of a BiCGStab solve, alpha from nb <= 256 partials of (r^, v)
+// the same for s = r - alpha v of a BiCGStab solve, alpha from nb <= kBicgPartials partials of (r^, v)
 void launch_patch_apply_s(cmg_ctx* c, const BicgVec& k, const double* part, int nb, double* z, const PatchSets& ps);
 // A x = b, right preconditioned with the context's preconditioner (built by the caller);
 // zero_guess: x starts at zero whatever it holds

@@ -39,6 +39,8 @@ namespace cmg {
 namespace {
 
 constexpr int kFusedRhs = 1024;     // components of r_c that the product's workgroups sum themselves
+constexpr int kCoarseRows = 2048;   // and at most
+constexpr int kRhsAhead = 8;
 constexpr int kTile = 32;            // columns per elimination panel
 constexpr int kGalRows = 28;         // blocks of a row staged in LDS at a time
 constexpr int kGalPart = 8 * 9 * 64; // partial sums of one chunk: [corner][entry][lane]
@@ -303,8 +305,9 @@ __global__ __launch_bounds__(256) void k_coarse_rhs(CoarseGrid g, const double* 
 
 // z_c = A_c^{-1} r_c, one row per wave.  FUSED: every workgroup sums r_c itself, in chunk
 // order.  With more than kFusedRhs components that serial sum costs more than a launch of
-// its own: 990 components (20k-element LV) 7.5 us fused, 4.7 + 4.7 us with k_coarse_rhs;
-// 2,040 (200k) 34 us fused, 11.3 + 4.6 us
+// its own: 990 components (20k-element LV) 5.9 us fused, 4.7 + 4.7 us with k_coarse_rhs;
+// 2,040 (200k) 34 us fused, 9.0 + 4.7 us.  The inverse's row and eight partials at a time are
+// requested ahead (7.8 us fused and 11.4 + 4.7 us without).
 template <bool FUSED>
 __global__ __launch_bounds__(256) void k_coarse_solve(CoarseGrid g, const double* A, const double* rpart,
                                                       int64_t set_rpart, const double* rcg, double* zc,
@@ -320,24 +323,37 @@ __global__ __launch_bounds__(256) void k_coarse_solve(CoarseGrid g, const double
     A += set * g.set_A;
     zc += set * (int64_t)g.ld;
     const int n = 3 * g.nodes;
+    // the row of the inverse is requested before r_c is summed
+    constexpr int K = (FUSED ? kFusedRhs : kCoarseRows) / 64;
+    const int row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    const double* a = A + (int64_t)min(row, n - 1) * g.ld;
+    double ar[K];
+#pragma unroll
+    for (int u = 0; u < K; u++) ar[u] = lane + 64 * u < n ? a[lane + 64 * u] : 0.0;
     if (FUSED) {
         rpart += set * set_rpart;
         for (int d = (int)threadIdx.x; d < n; d += 256) {
-            const int I = d / 3, i = d - 3 * I, e1 = g.rptr[I + 1];
+            const int I = d / 3, i = d - 3 * I, e0 = g.rptr[I], e1 = g.rptr[I + 1];
             double s = 0.0;
-            for (int e = g.rptr[I]; e < e1; e++) s += rpart[3 * (int64_t)e + i];
+            for (int e = e0; e < e1; e += kRhsAhead) {   // loaded together, summed in order
+                double v[kRhsAhead];
+#pragma unroll
+                for (int u = 0; u < kRhsAhead; u++) v[u] = rpart[3 * (int64_t)min(e + u, e1 - 1) + i];
+#pragma unroll
+                for (int u = 0; u < kRhsAhead; u++)
+                    if (e + u < e1) s += v[u];
+            }
             rc[d] = s;
         }
     } else {
         for (int d = (int)threadIdx.x; d < n; d += 256) rc[d] = rcg[set * (int64_t)g.ld + d];
     }
-    const int row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
     __syncthreads();
     if (row >= n) return;
-    const double* a = A + (int64_t)row * g.ld;
     double s = 0.0;
-#pragma unroll 8
-    for (int c = lane; c < n; c += 64) s += a[c] * rc[c];
+#pragma unroll
+    for (int u = 0; u < K; u++)
+        if (lane + 64 * u < n) s += ar[u] * rc[lane + 64 * u];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) zc[row] = s;
@@ -419,6 +435,7 @@ int build_coarse(cmg_ctx* c, const double* X, const int32_t* elements) {
                     }
                 }
         map.swap(node);
+        if (nodes > target) return false;
         for (int64_t e = 0; e < E; e++) {
             int mn[3] = {1024, 1024, 1024}, mx[3] = {0, 0, 0};
             for (int q = 0; q < npe; q++) {
@@ -429,7 +446,7 @@ int build_coarse(cmg_ctx* c, const double* X, const int32_t* elements) {
             for (int d = 0; d < 3; d++)
                 if (mx[d] - mn[d] > 1) return false;
         }
-        return nodes <= target;
+        return true;
     };
     int good = 0, bad = 1;
     while (bad <= 512 && lay(bad)) {
