@@ -199,7 +199,7 @@ void bgather_tangent(cmg_batch* b) {
 }
 
 // z = P^-1 u of every set not in b->apply_skip (the Schwarz application of the CG)
-void batch_schwarz_apply(void* bb, const double* u, double* z) {
+void batch_schwarz_apply(void* bb, const double* u, double* z, double* part, int64_t part_ld) {
     cmg_batch* b = static_cast<cmg_batch*>(bb);
     PatchSets ps;
     ps.S = b->S;
@@ -210,6 +210,8 @@ void batch_schwarz_apply(void* bb, const double* u, double* z) {
     ps.y = b->sw_y.as<double>();
     ps.coarse = &b->coarse;
     ps.flags = b->apply_skip;
+    ps.dots = part;
+    ps.dots_ld = part_ld;
     launch_patch_apply(b->c, u, z, ps);
 }
 
@@ -541,7 +543,7 @@ int cmg_batch_create(cmg_ctx* c, int32_t n_sets, const cmg_material* materials, 
     CMG_TRY(alloc(b->flags, (size_t)S * 2 * sizeof(int32_t)));
     b->part_ld = std::max<int64_t>({(int64_t)batch_spmv_blocks(c->N, 16), 2 * (int64_t)batch_node_blocks(c->N),
                                     (int64_t)batch_dot_blocks(n)}) + 1;
-    CMG_TRY(alloc(b->part, (size_t)S * b->part_ld * sizeof(double)));
+    CMG_TRY(alloc(b->part, (size_t)S * (b->part_ld + 2 * batch_node_blocks(c->N)) * sizeof(double)));
     CMG_TRY(alloc(b->active, S * sizeof(int32_t)));
     CMG_TRY(alloc(b->corrupt, S * sizeof(int32_t)));
     CMG_TRY(alloc(b->rtol, S * sizeof(double)));
@@ -560,12 +562,14 @@ int cmg_batch_create(cmg_ctx* c, int32_t n_sets, const cmg_material* materials, 
     cg.rr = sc + S;
     cg.rr0 = sc + 2 * S;
     cg.alpha = sc + 3 * S;
-    cg.beta = sc + 4 * S;
+    cg.rz_next = sc + 4 * S;
     cg.tol2 = sc + 5 * S;
     cg.done = b->flags.as<int32_t>();
     cg.it = b->flags.as<int32_t>() + S;
     cg.part = b->part.as<double>();
     cg.part_ld = b->part_ld;
+    cg.part_rz_ld = 2 * (int64_t)batch_node_blocks(c->N);
+    cg.part_rz = cg.part + S * b->part_ld;
     // every set starts from the context's current configuration
     for (int i = 0; i < S; i++)
         CMG_HIP_CHECK(hipMemcpyAsync(b->nodes.as<double>() + i * n, c->nodes.p, n * sizeof(double),

@@ -3,6 +3,10 @@
 // Jacobi inverses).  Every launch covers all sets (blockIdx.y = set); the scalar
 // recurrences of the preconditioned conjugate gradient stay in device memory, so a
 // run of iterations needs no host synchronisation and can be captured as one graph.
+// The kernels that use a scalar sum its partials themselves, every workgroup in the same
+// order: a launch of one workgroup per set took 3 to 4 us, and there were three such per
+// iteration (eight sets of 5k elements: six launches and 38 us against nine and 46 us).  What a kernel reads is
+// never what its first workgroup writes: r.z goes to rz_next, which the next product commits.
 // Reductions are two-stage in a fixed order: results do not depend on timing.
 #include "batch_kernels.h"
 
@@ -26,10 +30,11 @@ template <typename VT, int LANES>
 __global__ __launch_bounds__(kThreads) void k_bcg_spmv_dot(int64_t N, const int64_t* rowptr, const int32_t* colind,
                                                            const VT* vals, int64_t set_vals, const double* p,
                                                            double* q, int64_t n, const int32_t* done,
-                                                           double* partial, int nb) {
+                                                           double* partial, int nb, double* rz, const double* rz_next) {
     __shared__ double sh[4];
     const int64_t set = blockIdx.y;
     if (done[set]) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) rz[set] = rz_next[set];
     vals += set * set_vals;
     p += set * n;
     q += set * n;
@@ -105,14 +110,25 @@ __global__ __launch_bounds__(kThreads) void k_bcg_alpha(BatchCG cg, int nb) {
 }
 
 // x += alpha p, r -= alpha q, z = D^-1 r; partial r.z and r.r (one node per thread).
-// Without dinv only x and r (z then comes from the preconditioner, the partials from k_bcg_rz).
+// Without dinv only x and r (z and the partials then come from the preconditioner).
+// alpha from the product's nb partials, or from k_bcg_alpha (nb = 0).
 __global__ __launch_bounds__(kThreads) void k_bcg_update(BatchCG cg, int64_t N, const double* dinv, int nb) {
     __shared__ double sh[4];
     const int64_t set = blockIdx.y;
     if (cg.done[set]) return;
     const int64_t n = 3 * N;
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    const double al = cg.alpha[set];
+    double al;
+    if (nb) {
+        const double pq = reduce_partials(cg.part + set * cg.part_ld, nb, 1, 0, sh);
+        if (!(pq > 0.0 && isfinite(pq))) {   // the operator is not positive definite on p
+            if (blockIdx.x == 0 && threadIdx.x == 0) cg.done[set] = 2;
+            return;
+        }
+        al = cg.rz[set] / pq;
+    } else {
+        al = cg.alpha[set];
+    }
     if (!dinv) {
         if (i < N) {
             double* x = cg.x + set * n + 3 * i;
@@ -153,17 +169,17 @@ __global__ __launch_bounds__(kThreads) void k_bcg_update(BatchCG cg, int64_t N, 
     const double trz = block_sum256(rz, sh);
     const double trr = block_sum256(rr, sh);
     if (threadIdx.x == 0) {
-        double* part = cg.part + set * cg.part_ld + 2 * blockIdx.x;
+        double* part = cg.part_rz + set * cg.part_rz_ld + 2 * blockIdx.x;
         part[0] = trz;
         part[1] = trr;
     }
 }
 
-// partial r.z and r.r after the preconditioner wrote z (p = z as well when init)
-__global__ __launch_bounds__(kThreads) void k_bcg_rz(BatchCG cg, int64_t N, const int32_t* active, bool init) {
+// p = z, partial r.z and r.r of the active sets after the preconditioner wrote z
+__global__ __launch_bounds__(kThreads) void k_bcg_start(BatchCG cg, int64_t N, const int32_t* active) {
     __shared__ double sh[4];
     const int64_t set = blockIdx.y;
-    if (init ? !active[set] : cg.done[set] != 0) return;
+    if (!active[set]) return;
     const int64_t n = 3 * N;
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     double rz = 0.0, rr = 0.0;
@@ -172,7 +188,7 @@ __global__ __launch_bounds__(kThreads) void k_bcg_rz(BatchCG cg, int64_t N, cons
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const double rv = cg.r[o + c], zc = cg.z[o + c];
-            if (init) cg.p[o + c] = zc;
+            cg.p[o + c] = zc;
             rz += rv * zc;
             rr += rv * rv;
         }
@@ -180,38 +196,33 @@ __global__ __launch_bounds__(kThreads) void k_bcg_rz(BatchCG cg, int64_t N, cons
     const double trz = block_sum256(rz, sh);
     const double trr = block_sum256(rr, sh);
     if (threadIdx.x == 0) {
-        double* part = cg.part + set * cg.part_ld + 2 * blockIdx.x;
+        double* part = cg.part_rz + set * cg.part_rz_ld + 2 * blockIdx.x;
         part[0] = trz;
         part[1] = trr;
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_bcg_beta(BatchCG cg, int nb) {
+// beta from the nb partials of r.z and r.r, p = z + beta p unless the set has converged
+__global__ __launch_bounds__(kThreads) void k_bcg_p(BatchCG cg, int64_t n, int nb) {
     __shared__ double sh[4];
-    const int set = blockIdx.x;
-    if (cg.done[set]) return;
-    const double* part = cg.part + (int64_t)set * cg.part_ld;
-    double t2[2];
-    reduce_partials_k<2>(part, nb, sh, t2);
-    const double rz = t2[0], rr = t2[1];
-    if (threadIdx.x == 0) {
-        cg.it[set] += 1;
-        cg.rr[set] = rr;
-        if (rr <= cg.tol2[set] || !isfinite(rr)) {
-            cg.done[set] = 1;
-        } else {
-            cg.beta[set] = rz / cg.rz[set];
-            cg.rz[set] = rz;
-        }
-    }
-}
-
-__global__ __launch_bounds__(kThreads) void k_bcg_p(BatchCG cg, int64_t n) {
     const int64_t set = blockIdx.y;
     if (cg.done[set]) return;
+    double t2[2];
+    reduce_partials_k<2>(cg.part_rz + set * cg.part_rz_ld, nb, sh, t2);
+    const double rz = t2[0], rr = t2[1];
+    const bool fin = rr <= cg.tol2[set] || !isfinite(rr);
+    const double b = rz / cg.rz[set];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        cg.it[set] += 1;
+        cg.rr[set] = rr;
+        if (fin)
+            cg.done[set] = 1;
+        else
+            cg.rz_next[set] = rz;
+    }
+    if (fin) return;
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
-    const double b = cg.beta[set];
     double* p = cg.p + set * n;
     p[i] = cg.z[set * n + i] + b * p[i];
 }
@@ -251,7 +262,7 @@ __global__ __launch_bounds__(kThreads) void k_bcg_init(BatchCG cg, int64_t N, co
     const double trz = block_sum256(rz, sh);
     const double trr = block_sum256(rr, sh);
     if (threadIdx.x == 0) {
-        double* part = cg.part + set * cg.part_ld + 2 * blockIdx.x;
+        double* part = cg.part_rz + set * cg.part_rz_ld + 2 * blockIdx.x;
         part[0] = trz;
         part[1] = trr;
     }
@@ -268,12 +279,12 @@ __global__ __launch_bounds__(kThreads) void k_bcg_init_reduce(BatchCG cg, int nb
         }
         return;
     }
-    const double* part = cg.part + (int64_t)set * cg.part_ld;
+    const double* part = cg.part_rz + (int64_t)set * cg.part_rz_ld;
     double t2[2];
     reduce_partials_k<2>(part, nb, sh, t2);
     const double rz = t2[0], rr = t2[1];
     if (threadIdx.x == 0) {
-        cg.rz[set] = rz;
+        cg.rz_next[set] = rz;
         cg.rr[set] = rr;
         cg.rr0[set] = rr;
         cg.tol2[set] = rtol[set] * rtol[set] * rr;
@@ -340,7 +351,7 @@ void launch_bcg_spmv_dot(const BatchCG& cg, int lanes, int64_t N, const int64_t*
     const int64_t n = 3 * N;
 #define CMG_SPMV(VT, L)                                                                                          \
     hipLaunchKernelGGL((k_bcg_spmv_dot<VT, L>), grid, dim3(kThreads), 0, s, N, rowptr, colind, (const VT*)vals, \
-                       set_vals, cg.p, cg.q, n, cg.done, cg.part, (int)cg.part_ld)
+                       set_vals, cg.p, cg.q, n, cg.done, cg.part, (int)cg.part_ld, cg.rz, cg.rz_next)
     if (fp32) {
         if (lanes == 4) CMG_SPMV(float, 4);
         else if (lanes == 16) CMG_SPMV(float, 16);
@@ -358,16 +369,19 @@ void launch_bcg_iteration(const BatchCG& cg, int lanes, int64_t N, const int64_t
                           const void* vals, bool fp32, int64_t set_vals, const double* dinv, hipStream_t s,
                           PrecondApply apply, void* apply_ctx) {
     launch_bcg_spmv_dot(cg, lanes, N, rowptr, colind, vals, fp32, set_vals, s);
-    hipLaunchKernelGGL(k_bcg_alpha, dim3(cg.S), dim3(kThreads), 0, s, cg, batch_spmv_blocks(N, lanes));
-    const int nbn = batch_node_blocks(N);
-    hipLaunchKernelGGL(k_bcg_update, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, apply ? nullptr : dinv, nbn);
-    if (apply) {
-        apply(apply_ctx, cg.r, cg.z);
-        hipLaunchKernelGGL(k_bcg_rz, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, (const int32_t*)nullptr, false);
+    // up to kSelfSummed partials every workgroup of the update sums them; beyond, that is more
+    // traffic than a launch is worth
+    constexpr int kSelfSummed = 1024;
+    int nb = batch_spmv_blocks(N, lanes);
+    if (nb > kSelfSummed) {
+        hipLaunchKernelGGL(k_bcg_alpha, dim3(cg.S), dim3(kThreads), 0, s, cg, nb);
+        nb = 0;
     }
-    hipLaunchKernelGGL(k_bcg_beta, dim3(cg.S), dim3(kThreads), 0, s, cg, nbn);
+    const int nbn = batch_node_blocks(N);
+    hipLaunchKernelGGL(k_bcg_update, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, apply ? nullptr : dinv, nb);
+    if (apply) apply(apply_ctx, cg.r, cg.z, cg.part_rz, cg.part_rz_ld);
     const int64_t n = 3 * N;
-    hipLaunchKernelGGL(k_bcg_p, dim3((unsigned)((n + kThreads - 1) / kThreads), cg.S), dim3(kThreads), 0, s, cg, n);
+    hipLaunchKernelGGL(k_bcg_p, dim3((unsigned)((n + kThreads - 1) / kThreads), cg.S), dim3(kThreads), 0, s, cg, n, nbn);
 }
 
 void launch_bcg_init(const BatchCG& cg, int64_t N, const double* b, const double* dinv, const double* rtol,
@@ -375,8 +389,8 @@ void launch_bcg_init(const BatchCG& cg, int64_t N, const double* b, const double
     const int nbn = batch_node_blocks(N);
     hipLaunchKernelGGL(k_bcg_init, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, b, apply ? nullptr : dinv, active);
     if (apply) {
-        apply(apply_ctx, cg.r, cg.z);
-        hipLaunchKernelGGL(k_bcg_rz, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, active, true);
+        apply(apply_ctx, cg.r, cg.z, nullptr, 0);
+        hipLaunchKernelGGL(k_bcg_start, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, active);
     }
     hipLaunchKernelGGL(k_bcg_init_reduce, dim3(cg.S), dim3(kThreads), 0, s, cg, nbn, rtol, active);
 }

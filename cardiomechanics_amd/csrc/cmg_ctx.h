@@ -197,6 +197,9 @@ struct PatchSets {
     double* y = nullptr;        // [S][sw_y_len] (the context's sw_y when null)
     CoarseBuf* coarse = nullptr;    // coarse matrices of the sets (the context's co_buf when null)
     const int32_t* flags = nullptr;
+    // per workgroup of 256 nodes and set: r.z and r.r of an application (null: not wanted)
+    double* dots = nullptr;
+    int64_t dots_ld = 0;
 };
 // coarse-grid correction (coarse.hip): grid nodes at most, the grid of a context with patches
 // (sets c->coarse), the inverse of A_c from the block values, z_c = A_c^-1 r_c

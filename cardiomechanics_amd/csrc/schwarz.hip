@@ -362,44 +362,74 @@ __global__ __launch_bounds__(256) void k_patch_apply(BicgVec kv, const double* a
 }
 
 // z[3n + c] = sum over the patches holding node n of their y rows, in patch order, plus the
-// coarse correction at the node (g.nodes > 0)
+// coarse correction at the node (g.nodes > 0); DOTS: and the workgroup's share of r.z and r.r
+template <bool DOTS>
 __global__ __launch_bounds__(256) void k_patch_gather(CoarseGrid g, const uint8_t* bcmask, const double* zc, int64_t N,
                                                       const int32_t* cptr, const int32_t* cpos, const double* y,
-                                                      double* z, int64_t set_y, int64_t set_vec, const int32_t* skip) {
+                                                      double* z, int64_t set_y, int64_t set_vec, const int32_t* skip,
+                                                      const double* r, double* dots, int64_t dots_ld) {
     const int64_t set = blockIdx.y;
     if (skip && skip[set]) return;
     y += set * set_y;
     z += set * set_vec;
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int k = cptr[n]; k < cptr[n + 1]; k++) {
-        const double* q = y + cpos[k];
-        s0 += q[0];
-        s1 += q[1];
-        s2 += q[2];
-    }
-    if (g.nodes > 0) {
-        const int32_t* ids = g.corner + 8 * (int64_t)g.cell[n];
-        const double fx = g.frac[3 * n], fy = g.frac[3 * n + 1], fz = g.frac[3 * n + 2];
-        const double* u = zc + set * (int64_t)g.ld;
-        double c0 = 0.0, c1 = 0.0, c2 = 0.0;
-#pragma unroll
-        for (int a = 0; a < 8; a++) {
-            const double w = ((a & 1) ? fx : 1.0 - fx) * ((a & 2) ? fy : 1.0 - fy) * ((a & 4) ? fz : 1.0 - fz);
-            const double* q = u + 3 * ids[a];
-            c0 += w * q[0];
-            c1 += w * q[1];
-            c2 += w * q[2];
+    if (!DOTS && n >= N) return;
+    double rz = 0.0, rr = 0.0;
+    if (n < N) {
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+        for (int k = cptr[n]; k < cptr[n + 1]; k++) {
+            const double* q = y + cpos[k];
+            s0 += q[0];
+            s1 += q[1];
+            s2 += q[2];
         }
-        const int m = bcmask[n];
-        s0 += (m & 1) ? 0.0 : c0;
-        s1 += (m & 2) ? 0.0 : c1;
-        s2 += (m & 4) ? 0.0 : c2;
+        if (g.nodes > 0) {
+            const int32_t* ids = g.corner + 8 * (int64_t)g.cell[n];
+            const double fx = g.frac[3 * n], fy = g.frac[3 * n + 1], fz = g.frac[3 * n + 2];
+            const double* u = zc + set * (int64_t)g.ld;
+            double c0 = 0.0, c1 = 0.0, c2 = 0.0;
+#pragma unroll
+            for (int a = 0; a < 8; a++) {
+                const double w = ((a & 1) ? fx : 1.0 - fx) * ((a & 2) ? fy : 1.0 - fy) * ((a & 4) ? fz : 1.0 - fz);
+                const double* q = u + 3 * ids[a];
+                c0 += w * q[0];
+                c1 += w * q[1];
+                c2 += w * q[2];
+            }
+            const int m = bcmask[n];
+            s0 += (m & 1) ? 0.0 : c0;
+            s1 += (m & 2) ? 0.0 : c1;
+            s2 += (m & 4) ? 0.0 : c2;
+        }
+        z[3 * n] = s0;
+        z[3 * n + 1] = s1;
+        z[3 * n + 2] = s2;
+        if (DOTS) {
+            const double* rv = r + set * set_vec + 3 * n;
+            const double zv[3] = {s0, s1, s2};
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                rz += rv[c] * zv[c];
+                rr += rv[c] * rv[c];
+            }
+        }
     }
-    z[3 * n] = s0;
-    z[3 * n + 1] = s1;
-    z[3 * n + 2] = s2;
+    if (DOTS) {
+        __shared__ double sh[2][4];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            rz += __shfl_xor(rz, o, 64);
+            rr += __shfl_xor(rr, o, 64);
+        }
+        if (threadIdx.x % 64 == 0) {
+            sh[0][threadIdx.x / 64] = rz;
+            sh[1][threadIdx.x / 64] = rr;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2)
+            dots[set * dots_ld + 2 * blockIdx.x + threadIdx.x] =
+                sh[threadIdx.x][0] + sh[threadIdx.x][1] + sh[threadIdx.x][2] + sh[threadIdx.x][3];
+    }
 }
 
 }  // namespace
@@ -564,9 +594,16 @@ void patch_apply(cmg_ctx* c, const BicgVec* kv, const double* apart, int na, con
     }
 #undef CMG_PAPPLY
     if (c->coarse) launch_coarse_solve(c, ps);
-    hipLaunchKernelGGL(k_patch_gather, dim3((unsigned)((c->N + 255) / 256), ps.S), dim3(256), 0, c->stream, g, bc,
-                       cb.zc.as<double>(), c->N, c->sw_cptr.as<int32_t>(), c->sw_cpos.as<int32_t>(), y, z, ps.set_y,
-                       ps.set_vec, ps.flags);
+    const dim3 node_grid((unsigned)((c->N + 255) / 256), ps.S);
+#define CMG_PGATHER(DOTS)                                                                                          \
+    hipLaunchKernelGGL(k_patch_gather<DOTS>, node_grid, dim3(256), 0, c->stream, g, bc, cb.zc.as<double>(), c->N,  \
+                       c->sw_cptr.as<int32_t>(), c->sw_cpos.as<int32_t>(), y, z, ps.set_y, ps.set_vec, ps.flags, r, \
+                       ps.dots, ps.dots_ld)
+    if (ps.dots)
+        CMG_PGATHER(true);
+    else
+        CMG_PGATHER(false);
+#undef CMG_PGATHER
 }
 
 }  // namespace
