@@ -381,7 +381,8 @@ void launch_bcg_iteration(const BatchCG& cg, int lanes, int64_t N, const int64_t
     hipLaunchKernelGGL(k_bcg_update, dim3(nbn, cg.S), dim3(kThreads), 0, s, cg, N, apply ? nullptr : dinv, nb);
     if (apply) apply(apply_ctx, cg.r, cg.z, cg.part_rz, cg.part_rz_ld);
     const int64_t n = 3 * N;
-    hipLaunchKernelGGL(k_bcg_p, dim3((unsigned)((n + kThreads - 1) / kThreads), cg.S), dim3(kThreads), 0, s, cg, n, nbn);
+    hipLaunchKernelGGL(k_bcg_p, dim3((unsigned)((n + kThreads - 1) / kThreads), cg.S), dim3(kThreads), 0, s, cg, n,
+                       nbn);
 }
 
 void launch_bcg_init(const BatchCG& cg, int64_t N, const double* b, const double* dinv, const double* rtol,

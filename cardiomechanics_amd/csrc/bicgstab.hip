@@ -268,7 +268,8 @@ __global__ __launch_bounds__(kThreads) void k_bicg_update(BicgVec k, int64_t n, 
     const int64_t i = 2 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
     if (i + 1 < n) {
         const double2 v = *reinterpret_cast<const double2*>(k.v + i), t = *reinterpret_cast<const double2*>(k.t + i);
-        const double2 ph = *reinterpret_cast<const double2*>(k.ph + i), s2 = *reinterpret_cast<const double2*>(k.sh + i);
+        const double2 ph = *reinterpret_cast<const double2*>(k.ph + i);
+        const double2 s2 = *reinterpret_cast<const double2*>(k.sh + i);
         double2 x = *reinterpret_cast<const double2*>(k.x + i), r = *reinterpret_cast<const double2*>(k.r + i);
         double2 p = *reinterpret_cast<const double2*>(k.p + i);
         x.x += alpha * ph.x + om * s2.x;
@@ -368,8 +369,8 @@ struct Launch {
         const int64_t* rp = c->rowptr.as<int64_t>();
         const int32_t* ci = c->colind.as<int32_t>();
 #define CMG_BICG(VT, G)                                                                                           \
-    hipLaunchKernelGGL((k_bicg_spmv<VT, G, DOTS>), grid, dim3(kThreads), 0, s, k, c->N, tiles, rp, ci, (const VT*)vals, \
-                       u, y, part)
+    hipLaunchKernelGGL((k_bicg_spmv<VT, G, DOTS>), grid, dim3(kThreads), 0, s, k, c->N, tiles, rp, ci,            \
+                       (const VT*)vals, u, y, part)
         if (c->fp32) {
             if (lanes == 16) CMG_BICG(float, 16);
             else CMG_BICG(float, 8);

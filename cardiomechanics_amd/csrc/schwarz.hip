@@ -262,7 +262,8 @@ __global__ __launch_bounds__(256) void k_patch_invert(int64_t n, const int32_t* 
 #pragma unroll
     for (int j = 0; j < ND; j++) {
         const int c = __builtin_amdgcn_readlane(perm, j);
-        if (j < nd && c < nd && row >= 0 && row < nd) out[((int64_t)(c / G) * nd + row) * G + c % G] = (IT)(a[j] * scale);
+        if (j < nd && c < nd && row >= 0 && row < nd)
+            out[((int64_t)(c / G) * nd + row) * G + c % G] = (IT)(a[j] * scale);
     }
     for (int c = nd; c < (nd + G - 1) / G * G; c++)   // columns past nd are zero
         if (lane < nd) out[((int64_t)(c / G) * nd + lane) * G + c % G] = (IT)0;

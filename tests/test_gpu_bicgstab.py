@@ -77,13 +77,16 @@ def test_iterates_match_recurrence(order, n, precision):
 
 @pytest.mark.parametrize("pc", [1, 2], ids=["block_jacobi", "schwarz"])
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
-@pytest.mark.parametrize("size", [700, 50_000], ids=["one_row_group", "four_row_groups"])
+@pytest.mark.parametrize("size", [700, 9_000, 20_000, 30_000, 50_000])
 def test_true_residual_of_converged_solve(size, precision, pc):
-    """50,000 elements have more than 65,536 nodes, where a workgroup takes four row groups."""
+    """Row groups per workgroup of the product: one, two, four with 1,024 partials at most, one with
+    more of them, and four with more of them from 65,536 nodes on."""
     mesh = M.lv_mesh(size)
     rng = np.random.default_rng(6)
     with MechanicsContext(mesh, [MT.lv_holzapfel()], preconditioner=pc, precision=precision) as ctx:
-        assert size < 50_000 or ctx.n_dofs > 3 * 65_536
+        nodes = ctx.n_dofs // 3
+        assert {700: nodes < 8192, 9_000: 8192 < nodes < 16_384, 20_000: 24_576 < nodes < 32_768,
+                30_000: 32_768 < nodes < 65_536, 50_000: nodes > 65_536}[size]
         vals, A = system(ctx, mesh)
         b = A @ rng.normal(size=ctx.n_dofs)
         x, st = ctx.linear_solve(vals, b, rtol=1e-6)
