@@ -20,17 +20,17 @@ sys.path.insert(0, ROOT)
 
 import numpy as np  # noqa: E402
 
-# algorithmic HBM bytes per element (residual + analytic tangent): inputs 1548 B
-# (conn 40 + coordinates 240 + dN/dX 960 + bases 288 + scalars 20) + outputs
+# algorithmic HBM bytes per element (residual + analytic tangent): inputs 1004 B
+# (conn 40 + coordinates 240 + reference gradients 416 + bases 288 + scalars 20) + outputs
 # f 240 + K_e 7200 (FP64) / 3600 (FP32 values)
-BYTES_PER_ELEM = {0: 1548 + 240 + 7200, 1: 1548 + 240 + 3600}
+BYTES_PER_ELEM = {0: 1004 + 240 + 7200, 1: 1004 + 240 + 3600}
 FLOPS_PER_ELEM = 42_700
-# residual only: inputs 1548 B + f 240 B
-RES_BYTES_PER_ELEM = 1548 + 240
-# measured HBM bytes per element of the default kernels (FP64 variant 6, mixed variant 5):
+# residual only: inputs 1004 B + f 240 B
+RES_BYTES_PER_ELEM = 1004 + 240
+# measured HBM bytes per element of the default kernels (variant 6):
 # rocprofv3 FETCH_SIZE + WRITE_SIZE per dispatch, calibrated on a copy kernel of known size,
-# on the 200,340-element LV (profiles/element_residual_tangent_lv200k_fp64.md)
-TRAFFIC_PER_ELEM = {0: 8_881, 1: 5_263}
+# on the 200,340-element LV (profiles/kernels_by_call.md)
+TRAFFIC_PER_ELEM = {0: 8_327, 1: 4_695}
 HBM_PEAK = 8.0e12
 
 
@@ -244,7 +244,7 @@ def main():
                                   "re-measured in this run",
                 "bytes_per_element": BYTES_PER_ELEM[prec], "kernel": f"k_residual_tangent variant {best}",
                 "fp64_flops_per_s": FLOPS_PER_ELEM * E / (kernel_ms * 1e-3)}
-    # residual only (the line-search / convergence-check evaluation): 1,788 B and 3,160 flops per element
+    # residual only (the line-search / convergence-check evaluation): 1,244 B and 3,160 flops per element
     res_ms, _ = time_kernel(ctx, args.steps, args.warmup, tangent=0)
     residual_only = {"elem_per_s": E / (res_ms * 1e-3), "ms": res_ms, "bytes_per_element": RES_BYTES_PER_ELEM,
                      "achieved_GBps": RES_BYTES_PER_ELEM * E / (res_ms * 1e-3) / 1e9,
