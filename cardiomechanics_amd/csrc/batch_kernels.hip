@@ -5,8 +5,9 @@
 // run of iterations needs no host synchronisation and can be captured as one graph.
 // The kernels that use a scalar sum its partials themselves, every workgroup in the same
 // order: a launch of one workgroup per set took 3 to 4 us, and there were three such per
-// iteration (eight sets of 5k elements: six launches and 38 us against nine and 46 us).  What a kernel reads is
-// never what its first workgroup writes: r.z goes to rz_next, which the next product commits.
+// iteration (eight sets of 5k elements: six launches and 38 us against nine and 46 us).  A scalar
+// that the first workgroup stores is never one that the others read: r.z goes to rz_next, which
+// the next product commits.  The exception is the set's flag, see set_done.
 // Reductions are two-stage in a fixed order: results do not depend on timing.
 #include "batch_kernels.h"
 
@@ -23,6 +24,18 @@ __device__ __forceinline__ double block_sum256(double v, double* sh) {
     if (l == 0) sh[w] = v;
     __syncthreads();
     return sh[0] + sh[1] + sh[2] + sh[3];
+}
+
+// The set's flag, for a kernel whose first workgroup may set it: one thread reads it for its
+// whole workgroup, so that a flag set meanwhile stops all of its waves or none.  (Waves that
+// each read it could part ways before a sum over the workgroup, which then lacks the share
+// of those that left.)  The workgroups may differ: each finds the same verdict in its own
+// sums and leaves the set's vectors alone.
+__device__ __forceinline__ bool set_done(const int32_t* done, int64_t set) {
+    __shared__ int32_t flag;
+    if (threadIdx.x == 0) flag = done[set];
+    __syncthreads();
+    return flag != 0;
 }
 
 // q = A p for one set, LANES lanes per block row, plus the block's share of p . q
@@ -115,7 +128,7 @@ __global__ __launch_bounds__(kThreads) void k_bcg_alpha(BatchCG cg, int nb) {
 __global__ __launch_bounds__(kThreads) void k_bcg_update(BatchCG cg, int64_t N, const double* dinv, int nb) {
     __shared__ double sh[4];
     const int64_t set = blockIdx.y;
-    if (cg.done[set]) return;
+    if (set_done(cg.done, set)) return;
     const int64_t n = 3 * N;
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     double al;
@@ -206,7 +219,7 @@ __global__ __launch_bounds__(kThreads) void k_bcg_start(BatchCG cg, int64_t N, c
 __global__ __launch_bounds__(kThreads) void k_bcg_p(BatchCG cg, int64_t n, int nb) {
     __shared__ double sh[4];
     const int64_t set = blockIdx.y;
-    if (cg.done[set]) return;
+    if (set_done(cg.done, set)) return;
     double t2[2];
     reduce_partials_k<2>(cg.part_rz + set * cg.part_rz_ld, nb, sh, t2);
     const double rz = t2[0], rr = t2[1];
