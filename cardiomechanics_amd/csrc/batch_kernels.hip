@@ -223,13 +223,13 @@ __global__ __launch_bounds__(kThreads) void k_bcg_p(BatchCG cg, int64_t n, int n
     double t2[2];
     reduce_partials_k<2>(cg.part_rz + set * cg.part_rz_ld, nb, sh, t2);
     const double rz = t2[0], rr = t2[1];
-    const bool fin = rr <= cg.tol2[set] || !isfinite(rr);
+    const int fin = rr <= cg.tol2[set] ? 1 : !isfinite(rr) ? 2 : 0;
     const double b = rz / cg.rz[set];
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         cg.it[set] += 1;
         cg.rr[set] = rr;
         if (fin)
-            cg.done[set] = 1;
+            cg.done[set] = fin;
         else
             cg.rz_next[set] = rz;
     }
@@ -302,7 +302,8 @@ __global__ __launch_bounds__(kThreads) void k_bcg_init_reduce(BatchCG cg, int nb
         cg.rr0[set] = rr;
         cg.tol2[set] = rtol[set] * rtol[set] * rr;
         cg.it[set] = 0;
-        cg.done[set] = (rr == 0.0 || !(rz > 0.0)) ? 1 : 0;
+        // a right-hand side that the preconditioner turns round (or that is not finite) is no solution
+        cg.done[set] = rr == 0.0 ? 1 : !(rz > 0.0) || !isfinite(rr) ? 2 : 0;
     }
 }
 

@@ -1,6 +1,7 @@
-// The update of the parameter batch's conjugate gradient (batch_kernels.hip) where a set breaks
-// down, on the CPU model of workgroups: one wave of a workgroup reads the set's flag after
-// the launch's first workgroup has set it, the others before.
+// The parameter batch's conjugate gradient (batch_kernels.hip) where a set breaks down, on the
+// CPU model of workgroups: in the update, where one wave of a workgroup reads the set's flag
+// after the launch's first workgroup has set it, the others before; at the start and at
+// the end of an iteration, by the flag that the set is left with.
 #include "batch_kernels.hip"
 
 #include <cstdio>
@@ -46,5 +47,31 @@ int main() {
         std::printf("late wave %d: set 0 iterations %d, set 1 flag %d, entries changed %d\n", wave, it[0], done[1], moved);
         wrong += it[0] != 1 || done[1] != 2 || moved != 0 || x[0] == 0.0;
     }
+    // the start: solved (no right-hand side), turned round by the preconditioner, not finite
+    auto start = [&](double rhs, double pre) {
+        for (int64_t k = 0; k < N; k++)
+            for (int c = 0; c < 3; c++) b[3 * k + c] = rhs, dinv[9 * k + 4 * c] = pre;
+        launch_bcg_init(cg, N, b.data(), dinv.data(), rtol.data(), active.data(), nullptr);
+        std::printf("right-hand side %g, preconditioner %g: flag %d\n", rhs, pre, done[0]);
+        return done[0];
+    };
+    wrong += start(0.0, 1.0) != 1;
+    wrong += start(1.0, 1.0) != 0;
+    wrong += start(1.0, -1.0) != 2;
+    wrong += start(1.0, 0.0) != 2;
+    wrong += start(NAN, 1.0) != 2;
+    wrong += start(1e200, 1.0) != 2;
+    // the end of an iteration from the products r.z and r.r: converged, running, not finite
+    auto end = [&](double rr) {
+        start(1.0, 1.0);
+        for (int k = 0; k < batch_node_blocks(N); k++) part_rz[2 * k] = 1.0, part_rz[2 * k + 1] = rr;
+        model::launch(dim3(1, 1), dim3(kThreads), [&] { k_bcg_p(cg, n, batch_node_blocks(N)); });
+        std::printf("r.r %g: flag %d\n", rr, done[0]);
+        return done[0];
+    };
+    wrong += end(1e-12) != 1;
+    wrong += end(1.0) != 0;
+    wrong += end(INFINITY) != 2;
+    wrong += end(NAN) != 2;
     return wrong;
 }

@@ -1,5 +1,6 @@
 """The batch's conjugate gradient kernels on a CPU model of workgroups (tests/host/model): a
-set that breaks down keeps its iterate whatever the order in which wavefronts see its flag."""
+set that breaks down keeps its iterate whatever the order in which wavefronts see its flag,
+and only a solved set is left with the flag of one."""
 import os
 import subprocess
 
@@ -7,7 +8,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "cardiomechanics_amd", "csrc")
 
 
-def test_breakdown_seen_by_some_waves_only(tmp_path):
+def test_breakdown_and_flags(tmp_path):
     exe = tmp_path / "cg_breakdown"
     subprocess.check_call(["g++", "-O1", "-std=c++17", "-pthread", "-Wno-unknown-pragmas", "-x", "c++",
                            os.path.join(ROOT, "tests", "host", "cg_breakdown.cpp"),
