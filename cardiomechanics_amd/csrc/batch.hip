@@ -279,9 +279,10 @@ int build_graph(cmg_batch* b) {
     return CMG_SUCCESS;
 }
 
-// CG on the active sets (flags already uploaded): delta = A^-1 rhs to rtol[s]; done[s] = 2
-// where it broke down
-int bcg_run(cmg_batch* b, const std::vector<double>& rtol, std::vector<int32_t>& its, std::vector<int32_t>& done) {
+// CG on the active sets (flags already uploaded): delta = A^-1 rhs to rtol[s] in at most maxit
+// iterations (whole replays); done[s] = 2 where it broke down
+int bcg_run(cmg_batch* b, const std::vector<double>& rtol, int maxit, std::vector<int32_t>& its,
+            std::vector<int32_t>& done) {
     cmg_ctx* c = b->c;
     hipStream_t s = c->stream;
     const int S = b->S;
@@ -305,7 +306,7 @@ int bcg_run(cmg_batch* b, const std::vector<double>& rtol, std::vector<int32_t>&
         CMG_HIP_CHECK(hipStreamSynchronize(s));
         bool all = true;
         for (int i = 0; i < S; i++) all = all && b->h_int[S + i] != 0;
-        if (all || total >= c->opt.krylov_maxit) break;
+        if (all || total >= maxit) break;
     }
     CMG_HIP_CHECK(hipGetLastError());
     done.assign(b->h_int + S, b->h_int + 2 * S);
@@ -313,22 +314,33 @@ int bcg_run(cmg_batch* b, const std::vector<double>& rtol, std::vector<int32_t>&
     return CMG_SUCCESS;
 }
 
-// bcg_run on the sets flagged `solve`; sets that break down with the coarse correction (it
+// bcg_run on the sets flagged `solve`.  Sets that break down with the coarse correction (it
 // finds the negative directions of an indefinite tangent at once) are solved again without it
+// in the iterations that are left; those whose coarse matrix was found indefinite at its setup
+// had no correction, so their second solve would be the first one again.
 int bcg_solve(cmg_batch* b, const std::vector<double>& rtol, const std::vector<int32_t>& solve,
               std::vector<int32_t>& its) {
-    const int S = b->S;
+    hipStream_t s = b->c->stream;
+    const int S = b->S, maxit = b->c->opt.krylov_maxit;
     std::vector<int32_t> done;
     CMG_TRY(upload_flags(b, solve));
-    CMG_TRY(bcg_run(b, rtol, its, done));
+    CMG_TRY(bcg_run(b, rtol, maxit, its, done));
     if (!b->schwarz || !b->c->coarse) return CMG_SUCCESS;
     std::vector<int32_t> again(S, 0), its2;
     for (int i = 0; i < S; i++) again[i] = solve[i] && done[i] == 2;
     if (!any(again)) return CMG_SUCCESS;
+    CMG_HIP_CHECK(hipMemcpyAsync(b->h_int + S, b->coarse.bad.p, S * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    CMG_HIP_CHECK(hipStreamSynchronize(s));
+    int used = 0;
+    for (int i = 0; i < S; i++) {
+        again[i] = again[i] && !b->h_int[S + i];
+        if (again[i]) used = std::max(used, (int)its[i]);
+    }
+    if (!any(again) || used >= maxit) return CMG_SUCCESS;
     for (int i = 0; i < S; i++)
-        if (again[i]) launch_fill_int(1, 1, b->coarse.bad.as<int>() + i, b->c->stream);
+        if (again[i]) launch_fill_int(1, 1, b->coarse.bad.as<int>() + i, s);
     CMG_TRY(upload_flags(b, again));
-    CMG_TRY(bcg_run(b, rtol, its2, done));
+    CMG_TRY(bcg_run(b, rtol, maxit - used, its2, done));
     for (int i = 0; i < S; i++)
         if (again[i]) its[i] += its2[i];
     return CMG_SUCCESS;

@@ -5,6 +5,9 @@ recurrence in numpy where it breaks down.  It must not depend on the order in wh
 launch's workgroups find the breakdown, so the same step also gives the same bits twice."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
+
+from test_gpu_coarse import background_grid, patches
 
 from cardiomechanics_amd import materials as MT
 from cardiomechanics_amd import mesh as M
@@ -88,3 +91,49 @@ def test_update_of_a_broken_down_set_is_the_iterate_before_it(order, n):
         assert its == want
         # another order of the same sums may lose a hundred times what numpy's loses
         assert abs(step - norm) <= (100 * lost + 1e-13) * norm
+
+
+def schwarz(mesh, A):
+    """the vertex-patch preconditioner without and with the coarse correction; the smallest eigenvalue of
+    the coarse matrix"""
+    inv = []
+    for nodes in patches(mesh.elements, np.unique(mesh.elements[:, :4])):
+        d = (3 * nodes[:, None] + np.arange(3)).ravel()
+        inv.append((d, np.linalg.inv(A[d][:, d].toarray())))
+    free = np.ones(3 * mesh.n_nodes)
+    for c in range(3):
+        free[c::3][(mesh.bc >> c) & 1 == 1] = 0.0
+    P = sp.diags(free) @ sp.kron(background_grid(mesh.coords, mesh.elements, min(340, len(inv) // 4)), sp.eye(3)).tocsr()
+    Ac = (P.T @ A @ P).toarray()
+    keep = np.diag(Ac) > 0
+    P, Ac = P[:, keep], Ac[np.ix_(keep, keep)]
+    Ai = np.linalg.inv(Ac)
+
+    def one(r):
+        z = np.zeros_like(r)
+        for d, Ap in inv:
+            z[d] += Ap @ r[d]
+        return z
+    return one, lambda r: one(r) + P @ (Ai @ (P.T @ r)), np.linalg.eigvalsh((Ac + Ac.T) / 2)[0]
+
+
+def test_second_solve_without_the_correction_only_where_the_first_had_it():
+    """Penalties for which the tangent is indefinite and the coarse matrix still positive (the
+    correction is on, the set is solved again without it) or not (it is off from the start)."""
+    mesh = M.cube_mesh(4)
+    penalties = (1e5, -815.0, -870.0)
+    sets = [MT.guccione(500.0, 8.0, 4.0, 8.0, K) for K in penalties]
+    stats, systems = first_step(mesh, sets, **OPTS)
+    for (step, its, _, _), (A, b), K in zip(stats, systems, penalties):
+        one, two, least = schwarz(mesh, A)
+        x, want, end = pcg(A, two if least > 0 else one, b, 0.1)
+        if K < 0:
+            assert end == BREAKDOWN and (least > 0) == (K == -815.0)
+            if least > 0:
+                x, more, end = pcg(A, one, b, 0.1)
+                assert end == BREAKDOWN and more > want > 0
+                want += more
+        print(f"K {K:g}: {its} iterations (numpy {want}), |delta| {step:.12e} (numpy {np.linalg.norm(x):.12e})", flush=True)
+        assert its == want
+        # iterates of at most nine iterations; a converged one is known to the forcing tolerance
+        assert abs(step - np.linalg.norm(x)) <= (1e-8 if K < 0 else 1e-2) * np.linalg.norm(x)
