@@ -9,6 +9,8 @@
 
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
+#include <cstring>
 #include <functional>
 #include <future>
 #include <memory>
@@ -169,25 +171,83 @@ inline void launch(dim3 grid, dim3 block, const std::function<void()>& kernel) {
     }
 }
 
+// launches between the begin and the end of a capture
+typedef std::vector<std::function<void()>> Graph;
+inline Graph* recording = nullptr;
+
 }  // namespace model
+
+typedef model::Graph *hipGraph_t, *hipGraphExec_t;
+constexpr hipError_t hipErrorNotReady = 600;
+constexpr int hipStreamCaptureModeThreadLocal = 1, hipHostMallocCoherent = 1, hipHostMallocMapped = 2;
+constexpr int hipMemcpyHostToDevice = 1;
+#define __HIP_MEMORY_SCOPE_SYSTEM 0
+#define __hip_atomic_store(p, v, order, scope) __atomic_store_n(p, v, order)
+inline hipError_t hipMalloc(void** p, size_t n) { return (*p = aligned_alloc(256, (n + 255) / 256 * 256)) ? 0 : 2; }
+inline hipError_t hipHostMalloc(void** p, size_t n, int) { return hipMalloc(p, n); }
+inline hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, int, hipStream_t) { return memcpy(to, from, n), 0; }
+inline hipError_t hipFree(void* p) { return free(p), 0; }
+inline hipError_t hipGetLastError() { return 0; }
+inline hipError_t hipStreamQuery(hipStream_t) { return 0; }
+inline hipError_t hipStreamBeginCapture(hipStream_t, int) { return model::recording = new model::Graph, 0; }
+inline hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+    *g = model::recording;
+    model::recording = nullptr;
+    return 0;
+}
+inline hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, void*, void*, size_t) {
+    return *e = new model::Graph(*g), 0;
+}
+inline hipError_t hipGraphDestroy(hipGraph_t g) { return delete g, 0; }
+inline hipError_t hipGraphExecDestroy(hipGraphExec_t g) { return delete g, 0; }
+inline hipError_t hipGraphLaunch(hipGraphExec_t g, hipStream_t) {
+    for (auto& f : *g) f();
+    return 0;
+}
+struct double2 {
+    double x, y;
+};
+inline int min(int a, int b) { return a < b ? a : b; }
+inline void __threadfence_system() {}
 
 #define blockIdx model::block_idx
 #define threadIdx model::thread_idx
 #define gridDim model::grid_dim
 #define blockDim model::block_dim
+// arguments are evaluated at the launch, so that a captured one can run later
+template <typename F, typename... A>
+void launch_kernel(dim3 grid, dim3 block, F kernel, A... args) {
+    std::function<void()> f = [=] { kernel(args...); };
+    if (model::recording)
+        model::recording->push_back([=] { model::launch(grid, block, f); });
+    else
+        model::launch(grid, block, f);
+}
 #define hipLaunchKernelGGL(kernel, grid, block, lds, stream, ...) \
-    model::launch(grid, block, [&] { kernel(__VA_ARGS__); })
+    launch_kernel(grid, block, [](auto... a) { kernel(a...); }, __VA_ARGS__)
 
 inline void __syncthreads() { model::wait(model::kBarrier); }
 
 template <typename T>
-T __shfl_xor(T v, int mask, int width) {
+T shuffle(T v, int to, int width) {
     static_assert(sizeof(T) <= sizeof(double), "one exchange slot per lane");
     model::Workgroup& g = *model::current;
-    const int t = g.at, lane = t % model::kWave, to = t - lane + ((lane / width) * width + ((lane % width) ^ mask));
+    const int t = g.at;
     g.exchange[t] = v;
     model::wait(width);   // the others' values are there when this wave comes round again
     const T r = (T)g.exchange[to];
     model::wait(width);
     return r;
+}
+
+template <typename T>
+T __shfl_xor(T v, int mask, int width) {
+    const int t = model::current->at;
+    return shuffle(v, t - t % width + ((t % width) ^ mask), width);
+}
+
+template <typename T>
+T __shfl_down(T v, int by, int width) {
+    const int t = model::current->at;
+    return shuffle(v, t % width + by < width ? t + by : t, width);
 }
