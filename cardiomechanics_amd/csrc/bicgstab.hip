@@ -249,12 +249,16 @@ __global__ __launch_bounds__(kThreads) void k_bicg_update(BicgVec k, int64_t n, 
     const double alpha = sc->alpha, rho = sc->rho;
     const double om = tt > 0.0 ? ts / tt : 0.0;
     const double rho_new = rhs - om * rht;
-    const double rr = fmax(ss - 2.0 * om * ts + om * om * tt, 0.0);
-    const int it = sc->it + 1;
+    const double rr = ss - 2.0 * om * ts + om * om * tt;
+    // sums that are not finite: x stays where the iteration found it, which then does not count
+    const bool lost = !isfinite(rr);
+    const int it = sc->it + (lost ? 0 : 1);
     int fin = 0;
-    if (rr <= sc->tol2)
+    if (lost)
+        fin = kBicgBreakdown;
+    else if (rr <= sc->tol2)
         fin = kBicgConverged;
-    else if (om == 0.0 || !(fabs(rho_new) > 0.0) || !isfinite(rho_new) || !isfinite(rr))
+    else if (om == 0.0 || !(fabs(rho_new) > 0.0) || !isfinite(rho_new))
         fin = kBicgBreakdown;
     else if (it >= sc->maxit)
         fin = kBicgMaxit;
@@ -265,6 +269,7 @@ __global__ __launch_bounds__(kThreads) void k_bicg_update(BicgVec k, int64_t n, 
         sc->fin = fin;
         bicg_publish(sc, k.host, it, fin);
     }
+    if (lost) return;
     const int64_t i = 2 * ((int64_t)blockIdx.x * kThreads + threadIdx.x);
     if (i + 1 < n) {
         const double2 v = *reinterpret_cast<const double2*>(k.v + i), t = *reinterpret_cast<const double2*>(k.t + i);
@@ -485,6 +490,7 @@ int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero
     }
     unsigned long long word = 0;
     int it0 = 0;   // iterations before the last (re)start
+    bool stuck = false;   // broken down in the first iteration after it: another one would do the same
     for (int restarts = 0;; restarts++) {
         CMG_TRY(wait_for(c, c->bicg_seq, 0, word));
         const double rn = std::sqrt(c->bicg_host->rr);
@@ -494,7 +500,7 @@ int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero
         st->converged = (word & 0xff) == kBicgConverged && c->bicg_host->rr <= c->bicg_host->tol2;
         if (rn == 0.0) st->converged = 1;
         // the residual just computed is the true one: converged, out of restarts or iterations, or lost
-        if ((word & 0xff) != 0 || restarts > 50) break;
+        if ((word & 0xff) != 0 || stuck || restarts > 50) break;
         int queued = it0;
         auto queue = [&]() -> int {
             CMG_HIP_CHECK(hipGraphLaunch(c->bicg_graph, s));
@@ -506,7 +512,9 @@ int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero
             CMG_TRY(queue());
             CMG_TRY(wait_for(c, c->bicg_seq, queued - kBicgChunk, word));
         } while ((word & 0xff) == 0);
-        it0 = (int)((word >> 8) & 0xffffffffu);
+        const int it = (int)((word >> 8) & 0xffffffffu);
+        stuck = (word & 0xff) == kBicgBreakdown && it == it0;
+        it0 = it;
         start(false, false);   // r = b - A x: confirms, or continues from x
     }
     CMG_HIP_CHECK(hipGetLastError());
