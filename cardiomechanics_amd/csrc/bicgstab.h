@@ -8,8 +8,10 @@ namespace cmg {
 
 constexpr int kBicgConverged = 1, kBicgBreakdown = 2, kBicgMaxit = 3;
 
-// fin ends the iteration (set by the last kernel of one, or by a breakdown in alpha), done
-// the updates that belong to it; *_next are what the next iteration starts from
+// fin ends the iterations, done the updates that belong to the one at hand; *_next are what the
+// next iteration starts from.  No launch reads a flag that it may set: the first product reads fin
+// and sets done, the launch that forms alpha the same, the second product reads done
+// and sets fin, and the update too.
 struct BicgScalars {
     double rho, rho_next, alpha, tol2;
     int32_t fin, done, it, it_next, maxit;
@@ -56,7 +58,6 @@ __device__ __forceinline__ bool bicg_alpha(const BicgVec& k, const double* part,
             k.sc->alpha = alpha;
         } else {
             k.sc->done = 1;
-            k.sc->fin = kBicgBreakdown;
             bicg_publish(k.sc, k.host, k.sc->it, kBicgBreakdown);
         }
     }

@@ -53,8 +53,12 @@ __global__ __launch_bounds__(kThreads) void k_bicg_spmv(BicgVec k, int64_t N, in
                                                         const int32_t* colind, const VT* vals, const double* u,
                                                         double* y, double* part) {
     BicgScalars* sc = k.sc;
-    if (sc->fin) {
-        if (DOTS == 1 && blockIdx.x == 0 && threadIdx.x == 0) sc->done = 1;
+    if (DOTS == 1 && sc->fin) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) sc->done = 1;
+        return;
+    }
+    if (DOTS != 1 && sc->done) {   // by the product before, or because alpha broke down
+        if (blockIdx.x == 0 && threadIdx.x == 0 && !sc->fin) sc->fin = kBicgBreakdown;
         return;
     }
     if (DOTS == 1 && blockIdx.x == 0 && threadIdx.x == 0) {

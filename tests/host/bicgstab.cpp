@@ -109,5 +109,39 @@ int main() {
         const cmg_solve_stats st = a.solve(b, x, 1e-9, 100);
         wrong += check(st.converged == 0 && st.iterations == 0 && a.c.bicg_seq == 2, "a breakdown in alpha, one restart");
     }
+    // alpha breaks down and one wave of a workgroup starts after workgroup 0 has ended: nothing is
+    // written, and the flags are those of a breakdown from the next product on
+    for (int wave = 0; wave < 4; wave++) {
+        System a(600, 4.0, -1.0, -1.5, 4.0);
+        const int nb = 75;
+        std::vector<double> part(nb, 1.0), v(7 * a.c.n, 1.0);
+        BicgScalars sc = {};
+        BicgHost host = {};
+        BicgVec k;
+        k.r = &v[0], k.v = &v[a.c.n], k.sh = &v[2 * a.c.n], k.rh = &v[3 * a.c.n], k.t = &v[4 * a.c.n];
+        k.sc = &sc, k.host = &host;
+        sc.rho = 1.0;
+        const unsigned blocks = 3;
+        auto form = [&] {
+            hipLaunchKernelGGL(k_bicg_s_bj, dim3(blocks), dim3(kThreads), 0, nullptr, k, a.c.N, a.c.dinv.as<double>(),
+                               part.data(), nb);
+        };
+        form();   // leaves a positive sum in the LDS
+        std::fill(v.begin() + 2 * a.c.n, v.begin() + 3 * a.c.n, 7.0);
+        std::fill(part.begin(), part.end(), 0.0);
+        model::plan.count = 0;
+        model::plan.launch = 0;
+        model::plan.late = dim3(1, 0);
+        model::plan.late_wave = wave;
+        form();
+        model::plan.launch = -1;
+        int moved = 0;
+        for (int64_t i = 0; i < a.c.n; i++) moved += v[2 * a.c.n + i] != 7.0;
+        hipLaunchKernelGGL((k_bicg_spmv<double, 16, kDots>), dim3((600 + 15) / 16), dim3(kThreads), 0, nullptr, k, a.c.N, 1,
+                           a.c.rowptr.as<int64_t>(), a.c.colind.as<int32_t>(), a.vals.data(), k.sh, k.t, part.data());
+        std::printf("late wave %d: entries written %d, done %d, fin %d\n", wave, moved, sc.done, sc.fin);
+        wrong += check(moved == 0 && sc.done == 1 && sc.fin == kBicgBreakdown && (host.word & 0xff) == kBicgBreakdown,
+                       "a breakdown in alpha seen late");
+    }
     return wrong;
 }
