@@ -35,7 +35,7 @@ struct cmg_batch {
     DevBuf vals, dinv;                             // [S][nnzb*9], [S][N*9]
     DevBuf sw_inv, sw_y;                           // Schwarz: [S][sw_inv_len], [S][sw_y_len]
     CoarseBuf coarse;                              // coarse correction of the Schwarz preconditioner
-    bool schwarz = false;
+    bool schwarz = false, use_coarse = false;
     const int32_t* apply_skip = nullptr;           // sets the Schwarz application skips
     DevBuf cg_r, cg_z, cg_p, cg_q;                 // [S][n]
     DevBuf sc;                                     // CG scalars: 6 doubles per set
@@ -185,6 +185,7 @@ void bgather_tangent(cmg_batch* b) {
         ps.set_inv = c->sw_inv_len;
         ps.inv = b->sw_inv.p;
         ps.coarse = &b->coarse;
+        ps.use_coarse = b->use_coarse;
         ps.flags = b->active.as<int32_t>();
         launch_patch_setup(c, b->vals.p, ps);
         return;
@@ -209,6 +210,7 @@ void batch_schwarz_apply(void* bb, const double* u, double* z, double* part, int
     ps.inv = b->sw_inv.p;
     ps.y = b->sw_y.as<double>();
     ps.coarse = &b->coarse;
+    ps.use_coarse = b->use_coarse;
     ps.flags = b->apply_skip;
     ps.dots = part;
     ps.dots_ld = part_ld;
@@ -325,7 +327,7 @@ int bcg_solve(cmg_batch* b, const std::vector<double>& rtol, const std::vector<i
     std::vector<int32_t> done;
     CMG_TRY(upload_flags(b, solve));
     CMG_TRY(bcg_run(b, rtol, maxit, its, done));
-    if (!b->schwarz || !b->c->coarse) return CMG_SUCCESS;
+    if (!b->use_coarse) return CMG_SUCCESS;
     std::vector<int32_t> again(S, 0), its2;
     for (int i = 0; i < S; i++) again[i] = solve[i] && done[i] == 2;
     if (!any(again)) return CMG_SUCCESS;
@@ -540,16 +542,16 @@ int cmg_batch_create(cmg_ctx* c, int32_t n_sets, const cmg_material* materials, 
     CMG_TRY(alloc(b->dinv, (size_t)S * c->N * 9 * sizeof(double)));
     if (c->schwarz) {
         // S sets of patch inverses (S x 548 MB in FP64 on the 200k LV): where they do not
-        // fit, the batch keeps block Jacobi
+        // fit, the batch keeps block Jacobi; where the coarse matrices do not, the patches alone
         b->schwarz = b->sw_inv.alloc((size_t)S * c->sw_inv_len * kt) &&
-                     b->sw_y.alloc((size_t)S * c->sw_y_len * sizeof(double)) &&
-                     (!c->coarse || b->coarse.alloc(c->co, S));
+                     b->sw_y.alloc((size_t)S * c->sw_y_len * sizeof(double));
         if (!b->schwarz) {
-            b->coarse.release();
             b->sw_inv.release();
             b->sw_y.release();
-            (void)hipGetLastError();   // the failed allocation is not an error of the batch
         }
+        b->use_coarse = b->schwarz && c->coarse && b->coarse.alloc(c->co, S);
+        if (!b->use_coarse) b->coarse.release();
+        (void)hipGetLastError();   // a failed allocation is not an error of the batch
     }
     CMG_TRY(alloc(b->sc, (size_t)S * 6 * sizeof(double)));
     CMG_TRY(alloc(b->flags, (size_t)S * 2 * sizeof(int32_t)));

@@ -196,6 +196,7 @@ struct PatchSets {
     void* inv = nullptr;        // [S][sw_inv_len] (the context's sw_inv when null)
     double* y = nullptr;        // [S][sw_y_len] (the context's sw_y when null)
     CoarseBuf* coarse = nullptr;    // coarse matrices of the sets (the context's co_buf when null)
+    bool use_coarse = true;         // false: without the correction, whatever the context has
     const int32_t* flags = nullptr;
     // per workgroup of 256 nodes and set: r.z and r.r of an application (null: not wanted)
     double* dots = nullptr;

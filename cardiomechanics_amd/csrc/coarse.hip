@@ -533,19 +533,23 @@ int build_coarse(cmg_ctx* c, const double* X, const int32_t* elements) {
     std::vector<int32_t> rslot(ridx.size());
     for (size_t e = 0; e < ridx.size(); e++) rslot[ridx[e]] = (int32_t)e;
     hipStream_t s = c->stream;
-    CMG_TRY(upload(c->co_pos, pos.data(), pos.size(), s));
-    CMG_TRY(upload(c->co_frac, frac.data(), frac.size(), s));
-    CMG_TRY(upload(c->co_order, order.data(), order.size(), s));
-    CMG_TRY(upload(c->co_cell, cell.data(), cell.size(), s));
-    CMG_TRY(upload(c->co_corner, corner.data(), corner.size(), s));
-    CMG_TRY(upload(c->co_chunk, chunk.data(), chunk.size(), s));
-    CMG_TRY(upload(c->co_rchunk, rchunk.data(), rchunk.size(), s));
-    CMG_TRY(upload(c->co_map, map.data(), map.size(), s));
-    CMG_TRY(upload(c->co_ijk, ijk.data(), ijk.size(), s));
-    CMG_TRY(upload(c->co_gptr, gptr.data(), gptr.size(), s));
-    CMG_TRY(upload(c->co_gidx, gidx.data(), gidx.size(), s));
-    CMG_TRY(upload(c->co_rptr, rptr.data(), rptr.size(), s));
-    CMG_TRY(upload(c->co_rslot, rslot.data(), rslot.size(), s));
+    auto put = [&]() -> int {
+        CMG_TRY(upload(c->co_pos, pos.data(), pos.size(), s));
+        CMG_TRY(upload(c->co_frac, frac.data(), frac.size(), s));
+        CMG_TRY(upload(c->co_order, order.data(), order.size(), s));
+        CMG_TRY(upload(c->co_cell, cell.data(), cell.size(), s));
+        CMG_TRY(upload(c->co_corner, corner.data(), corner.size(), s));
+        CMG_TRY(upload(c->co_chunk, chunk.data(), chunk.size(), s));
+        CMG_TRY(upload(c->co_rchunk, rchunk.data(), rchunk.size(), s));
+        CMG_TRY(upload(c->co_map, map.data(), map.size(), s));
+        CMG_TRY(upload(c->co_ijk, ijk.data(), ijk.size(), s));
+        CMG_TRY(upload(c->co_gptr, gptr.data(), gptr.size(), s));
+        CMG_TRY(upload(c->co_gidx, gidx.data(), gidx.size(), s));
+        CMG_TRY(upload(c->co_rptr, rptr.data(), rptr.size(), s));
+        CMG_TRY(upload(c->co_rslot, rslot.data(), rslot.size(), s));
+        return CMG_SUCCESS;
+    };
+    int rc = put();
     CoarseGrid& g = c->co;
     g.nodes = (int)ijk.size();
     g.ld = (3 * g.nodes + kTile - 1) / kTile * kTile;
@@ -568,8 +572,17 @@ int build_coarse(cmg_ctx* c, const double* X, const int32_t* elements) {
     g.gidx = c->co_gidx.as<int32_t>();
     g.rptr = c->co_rptr.as<int32_t>();
     g.rslot = c->co_rslot.as<int32_t>();
-    CMG_TRY(c->co_buf.alloc(g, 1) ? CMG_SUCCESS : fail("hipMalloc of the coarse matrix failed", CMG_ERR_NOMEM));
+    if (rc == CMG_SUCCESS && !c->co_buf.alloc(g, 1)) rc = CMG_ERR_NOMEM;
     CMG_HIP_CHECK(hipStreamSynchronize(s));
+    if (rc == CMG_ERR_NOMEM) {   // does not fit: the patches alone
+        for (DevBuf* b : {&c->co_pos, &c->co_frac, &c->co_order, &c->co_cell, &c->co_corner, &c->co_chunk, &c->co_rchunk,
+                          &c->co_map, &c->co_ijk, &c->co_gptr, &c->co_gidx, &c->co_rptr, &c->co_rslot})
+            b->release();
+        c->co_buf.release();
+        (void)hipGetLastError();   // the failed allocation is not an error of the context
+        return CMG_SUCCESS;
+    }
+    CMG_TRY(rc);
     c->coarse = true;
     return CMG_SUCCESS;
 }

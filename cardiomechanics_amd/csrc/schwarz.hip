@@ -564,7 +564,7 @@ void launch_patch_setup(cmg_ctx* c, const void* vals, const PatchSets& ps) {
         patch_setup(c, (const float*)vals, (float*)inv, ps);
     else
         patch_setup(c, (const double*)vals, (double*)inv, ps);
-    if (c->coarse) launch_coarse_setup(c, vals, ps);
+    if (c->coarse && ps.use_coarse) launch_coarse_setup(c, vals, ps);
 }
 
 namespace {
@@ -572,7 +572,8 @@ namespace {
 void patch_apply(cmg_ctx* c, const BicgVec* kv, const double* apart, int na, const double* r, double* z,
                  const PatchSets& ps) {
     const int ndm = (c->sw_nd_max + 3) / 4 * 4;   // whole groups
-    const CoarseGrid g = c->coarse ? c->co : CoarseGrid();
+    const bool coarse = c->coarse && ps.use_coarse;
+    const CoarseGrid g = coarse ? c->co : CoarseGrid();
     const CoarseBuf& cb = ps.coarse ? *ps.coarse : c->co_buf;
     const int64_t set_rpart = (int64_t)g.n_rchunk * 24;
     const uint8_t* bc = c->bcmask.as<uint8_t>();
@@ -594,7 +595,7 @@ void patch_apply(cmg_ctx* c, const BicgVec* kv, const double* apart, int na, con
         else CMG_PAPPLY(double, false);
     }
 #undef CMG_PAPPLY
-    if (c->coarse) launch_coarse_solve(c, ps);
+    if (coarse) launch_coarse_solve(c, ps);
     const dim3 node_grid((unsigned)((c->N + 255) / 256), ps.S);
 #define CMG_PGATHER(DOTS)                                                                                          \
     hipLaunchKernelGGL(k_patch_gather<DOTS>, node_grid, dim3(256), 0, c->stream, g, bc, cb.zc.as<double>(), c->N,  \
