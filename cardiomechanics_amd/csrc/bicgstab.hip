@@ -21,7 +21,8 @@
 // steps, ms): static step of the 1,296-element cube 13.3 / 18.5, Newmark step of the 20k LV
 // 24.0 / 31.0, of the 200k LV 320 / 328 in FP64 and 211 / 257 with the FP32 matrix (there
 // the product's time counts, see k_bicg_spmv).
-// All sums have a fixed order: a solve is reproducible bit for bit.
+// All sums have a fixed order: a context repeats a solve bit for bit (another one may have chosen
+// another layout for the product of the true residual, unless spmv_choice fixes it).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -40,7 +41,8 @@ constexpr int kBicgChunk = 4;     // iterations per graph launch
 // y = A u and the partial dot products of each workgroup's rows.  DOTS = 1: (rh, y);
 // DOTS = 5: the five sums with s = r - alpha v.
 //
-// Bound by the block values (572 MB on the 200k-element LV in FP64).  G lanes share a block
+// Bound by the block values (572 MB on the 200k-element LV in FP64): the first product moves
+// 744 MB at 5.2 TB/s, in FP32 453 MB at 5.6 TB/s, a large copy 5.9.  G lanes share a block
 // row.  FP64: three lanes per 3x3 block, one per block row, so a wave's load instruction
 // covers contiguous 24-byte pieces of 10 (G = 32) or 5 (G = 16) blocks per row; FP32: one
 // lane per block.  The loads of kUnroll steps (all of an average row) are issued before
@@ -440,7 +442,10 @@ int bicgstab(cmg_ctx* c, const void* vals, const double* b, double* x, bool zero
     L.lanes = (c->nnzb > 20 * c->N ? 2 : 1) * (c->fp32 ? 8 : 16);
     // row groups per workgroup: as few as leave kBicgPartials partials, up to four; meshes too
     // large for that have one or, where the chip is full anyway, four (20k-element LV, four
-    // groups: two reductions of 4.6 us less, the first product 2.6 us and the update 1.5 us more)
+    // groups: two reductions of 4.6 us less, the first product 2.6 us and the update 1.5 us more).
+    // Whole steps with one / four groups, iterations that move with the order of the sums among it
+    // (ms): FP64 40k elements 44.2 / 39.5, 50k (75,744 nodes) 57.5 / 57.8, 75k 84.0 / 88.5; mixed
+    // 31.8 / 31.7, 40.9 / 36.6, 54.3 / 56.2
     const int64_t groups = (c->N + kThreads / L.lanes - 1) / (kThreads / L.lanes);
     L.tiles = (int)((groups + kBicgPartials - 1) / kBicgPartials);
     if (L.tiles > 4) L.tiles = c->N > 65536 ? 4 : 1;

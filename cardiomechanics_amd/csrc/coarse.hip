@@ -25,7 +25,8 @@
 //                      the mesh does not resolve.  A clearly negative pivot marks an
 //                      indefinite tangent (soft parameter sets at an extrapolated guess):
 //                      the correction is then off (bad) until the next setup, and the
-//                      preconditioner is the one-level Schwarz.
+//                      preconditioner is the one-level Schwarz, as it is where these
+//                      buffers do not fit the device.
 // Per application: the restriction runs as extra workgroups of the patch launch,
 // k_coarse_solve sums the restriction partials and multiplies by the inverse, and the
 // patch gather adds P z_c.  All sums have a fixed order (no atomics).
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(256) void k_coarse_galerkin(CoarseGrid g, const int
         }
 #pragma unroll
         for (int q = 0; q < 9; q++)
-            if ((mask >> (q / 3)) & 1) t[q] = 0.0;   // constrained rows (their columns are zero already)
+            if ((mask >> (q / 3)) & 1) t[q] = 0.0;   // constrained rows (the assembly leaves zero columns)
 #pragma unroll
         for (int a = 0; a < 8; a++) {
             const double wr = ((a & 1) ? fx : 1.0 - fx) * ((a & 2) ? fy : 1.0 - fy) * ((a & 4) ? fz : 1.0 - fz);
@@ -372,7 +373,9 @@ int build_coarse(cmg_ctx* c, const double* X, const int32_t* elements) {
     // more grid nodes save iterations and cost inversion (2 n^3) and products (8 n^2 bytes):
     // twice as many pay from about 20,000 patches on (1 ms Newmark step, 340 / 680 nodes:
     // 20k-element LV, 4,400 patches, 29.9 / 32.0 ms; 200k-element LV, 39,375 patches,
-    // 320.9 / 301.4 ms)
+    // 320.9 / 301.4 ms).  In between either side may be ahead by 5 % (FP64, mixed: 50k elements,
+    // 10,610 patches, 58.4 / 57.1 and 36.5 / 38.5 ms; 75k 88.4 / 86.8 and 56.6 / 55.4; 100k, 21,175
+    // patches, 129.4 / 115.6 and 77.9 / 81.6)
     const int64_t most = c->sw_P < 20000 ? kCoarseMaxNodes : 2 * kCoarseMaxNodes;
     const int64_t target = std::min(most, c->sw_P / 4);
     if (target < 8) return CMG_SUCCESS;

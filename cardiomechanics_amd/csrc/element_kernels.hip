@@ -1643,7 +1643,8 @@ void launch_element_residual_tangent(int npe, bool fp32, const ElemArgs& a, hipS
 #define CMG_LAUNCH2(K) hipLaunchKernelGGL(K, dim3(nblk, a.n_sets), dim3(128), 0, s, a)
 // K_e larger than the 256 MB of the memory-side cache passes it by: the gather reads it from
 // memory anyway (200k elements 556 / 577 us in FP64, 348 / 369 mixed; 20k, which stay in it,
-// 59 / 56 and 47.8 / 45.0)
+// 59 / 56 and 47.8 / 45.0).  In between the line is not sharp: from 20k to 100k elements (72 to
+// 720 MB) a whole assembly differs by less than 1 % either way
 #define CMG_LAUNCH_T10(TT, L17, HALVES)                                                                            \
     hipLaunchKernelGGL((k_residual_tangent_t10<TT, L17, HALVES>), dim3(nblk2, a.n_sets), dim3(128 * HALVES), 0, s, a, \
                        (size_t)a.E * a.n_sets * 900 * sizeof(TT) > (size_t)256 << 20)
