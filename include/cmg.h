@@ -168,7 +168,8 @@ typedef struct cmg_options {
                                    context's first solve; 1-9: that layout without timing (1-3 one
                                    3x3 block per step at 4/8/16 lanes, 4-6 144-byte chunks at 4/8/16
                                    lanes, 7-9 the flat word stream at 16/32/64 lanes), so that two
-                                   contexts do the same arithmetic */
+                                   contexts do the same arithmetic.  GMRES and true residuals use
+                                   it; BiCGStab's own products have one layout */
 } cmg_options;
 
 typedef struct cmg_solve_stats {
