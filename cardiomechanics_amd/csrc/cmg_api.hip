@@ -1169,6 +1169,7 @@ int cmg_spmv(cmg_ctx* c, const double* values, const double* x, double* y) {
 
 int cmg_linear_solve(cmg_ctx* c, const double* values, const double* b, double* x, double rtol, cmg_solve_stats* st) {
     if (!c || !values || !b || !x) return fail("cmg_linear_solve: null argument");
+    CMG_HIP_CHECK(hipSetDevice(c->device));   // the first solve sets up its workspace
     const size_t vb = c->n * sizeof(double);
     const size_t vbytes = (size_t)c->nnzb * 9 * (c->fp32 ? sizeof(float) : sizeof(double));
     CMG_HIP_CHECK(hipMemcpyAsync(c->vals.p, values, vbytes, hipMemcpyHostToDevice, c->stream));
